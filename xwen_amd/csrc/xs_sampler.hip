@@ -64,6 +64,10 @@
 #include "xs_host.h"
 
 #define XS_DEV __device__ __forceinline__
+// A branch seldom taken and whose own speed does not matter: its code is laid
+// out away from the usual path (one row 12.5 -> 12.2 us), and unrolled less
+// (24 masked rows that take gather_survivors: 41 us without it there, 60 with).
+#define XS_RARE(...) __builtin_expect((__VA_ARGS__) ? 1 : 0, 0)
 
 typedef float v4f __attribute__((ext_vector_type(4)));
 
@@ -774,6 +778,7 @@ struct FinLds {
   uint64_t psel[KSEL];              // the candidate set in draw order: (p bits << 32) | ~id
   double expt[64];                  // kExpT, flattened
   uint32_t keys[GMAX * 64 * 4];     // published bound keys (more than 64 sub-records)
+  int32_t pref[64];                 // gather_survivors: a group's running entry counts
   uint32_t zmap[KSEL / 32];         // a whole short row: the ids with p > 0
   HeldLds held;
   BigStash big;
@@ -849,9 +854,13 @@ XS_DEV float q4(const v4f& q, int e) { return e == 0 ? q.x : e == 1 ? q.y : e ==
 
 // ---------------------------------------------------------------------------
 // Rare path of the chunk pass: more than CAPW of this wave's elements lie at
-// or above the chunk bound (ties at the bound, or a bound far below the
-// wave's values).  Writes the wave's exact K' best (logit desc, id asc)
-// elements: every key above a threshold key, then the lowest ids equal to it.
+// or above the chunk bound (a bound far below the wave's values, where a mask
+// leaves fewer finite lanes than K', or ties at it).  Stages the wave's
+// elements at or above a higher floor tf where they then fit, and returns
+// their count; each round reads them once more, where the 32-round search for
+// the exact threshold read them 33 times.  Otherwise (ovf) writes the wave's
+// exact K' best (logit desc, id asc) elements to its sub-record: every key
+// above a threshold key, then the lowest ids equal to it.
 // The threshold is the bound when fewer than K' keys lie strictly above it,
 // else the wave's K'-th largest key (bisection).  Elements that are -inf or
 // NaN never become candidates.  Re-reads the wave's elements from memory (the
@@ -868,7 +877,7 @@ struct ChunkCtl {
 
 template <bool HAS_MASK, bool HAS_CTL, bool LOC>
 XS_DEV int wave_overflow(const float* rowp, const uint32_t* mrow, int s0, int ns, int enc,
-                         uint64_t* sub, int nsp, int kp, uint32_t tk, const ChunkCtl& cc) {
+                         uint64_t* sub, int nsp, int kp, uint64_t* stg, float& tf, bool& ovf, const ChunkCtl& cc) {
   constexpr int H = SPC / 2;  // slots per round of loads
   const int tid = threadIdx.x;
   // Slots h*H .. h*H+H-1 of the wave's elements as the streaming pass saw
@@ -938,7 +947,40 @@ XS_DEV int wave_overflow(const float* rowp, const uint32_t* mrow, int s0, int ns
     }
     return wave_sumi(c);
   };
-  uint32_t eq = max(tk, fkey(-__FLT_MAX__));
+  // The K'-th largest of the staged elements is a higher floor, with K'
+  // elements at or above it: stage again from there, while it rises.
+  for (;;) {
+    wave_lds_sync();
+    uint32_t sk[CAPW / 64];
+#pragma unroll
+    for (int r = 0; r < CAPW / 64; r++) sk[r] = pk_key(stg[r * 64 + (tid & 63)]);
+    const float up = keyf(kth_largest<CAPW / 64>(sk, kp));
+    if (!(up > tf)) break;  // (ties at the floor)
+    tf = up;
+    wave_lds_sync();
+    int n = 0, pc = cc.p0;
+#pragma unroll 1
+    for (int h = 0; h < 2; h++) {
+      v4f xv[H];
+      load(h, xv, pc);
+#pragma unroll
+      for (int u = 0; u < H; u++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          const float x = q4(xv[u], e);
+          const bool hit = x >= tf;  // (tf is finite: never -inf, never NaN)
+          const uint64_t b = __ballot(hit);
+          if (b) {
+            const int pos = n + lanes_below(b);
+            if (hit && pos < CAPW) stg[pos] = pack(fkey(x), (uint32_t)((s0 + h * H + u) * SLOT + 4 * tid + e));
+            n += __popcll(b);
+          }
+        }
+    }
+    if (n <= CAPW) return n;
+  }
+  ovf = true;
+  uint32_t eq = fkey(tf);
   if (count(eq, true) >= kp) {
     uint32_t ans = 0;
 #pragma unroll 1
@@ -1379,9 +1421,159 @@ XS_DEV bool draw_settled(const float (&c)[R], float tot, float x, int idx, int k
 }
 
 // ---------------------------------------------------------------------------
+// The survivors of a row: its sub-records' entries at or above `fl_e`, into
+// F.list, at most SURV of them; returns their number M.  Whatever is left out
+// lies below K' entries that were kept: when the list fills, its K' best are
+// kept and fl_e rises to the last of them.
+//
+// The bound the published keys give is weak or absent on a row whose chunks
+// hold fewer finite (allowed) ids than K' asks for, or that has few chunks: a
+// small vocabulary, a mask of a few ranges.  Then up to CAPW entries of every
+// sub-record pass it.  When more entries may pass than the list holds, the
+// bound is first raised to the K'-th largest preloaded entry (E, EPRE of each
+// of the first 64 sub-records).  What is not preloaded is read 256 entries to
+// a round trip, whichever sub-records hold them: a lane finds its entry's
+// sub-record in the running counts (F.pref).
+//
+// Bound by latency on one wave.  The bitwise search over every entry that
+// stood here read a sub-record's entries one after another, 64 times over:
+// a call of 24 masked rows of 64,003 ids at top_k 50 went from 1,244 to 41 us
+// (with wave_overflow's rounds), 33 rows of 19,450 ids at top_k 100 from 375
+// us, C2 unchanged.
+template <bool LOC>
+XS_DEV int gather_survivors(const uint64_t* rowrec, int nsp, int nsub, int kp, const uint64_t (&E)[EPRE],
+                            int cnt0, bool srt0, uint64_t fl_e, FinLds& F) {
+  const int lane = lane_id();
+  const int G = (nsub + 63) >> 6;
+  // Lane l's preloaded entries above the floor, and how many of its
+  // sub-record's entries follow them (in a sorted one, flag 4, they end at the
+  // first below the floor).
+  bool ok[EPRE];
+  int c = 0, x = 0;
+  auto look = [&]() __attribute__((always_inline)) {
+    c = 0;
+#pragma unroll
+    for (int j = 0; j < EPRE; j++) {
+      ok[j] = j < cnt0 && E[j] >= fl_e;
+      c += ok[j] ? 1 : 0;
+    }
+    x = (srt0 && E[EPRE - 1] < fl_e) ? 0 : max(cnt0 - EPRE, 0);
+  };
+  look();
+  int incl = wave_incl_scan(c);
+  int M = (int)rdl((uint32_t)incl, 63);
+  bool more = __ballot(x > 0) != 0;
+  bool full = M > SURV;
+  if (more || full) full = M + wave_sumi(x) > SURV;
+  if (full) {
+    uint32_t key[EPRE];
+#pragma unroll
+    for (int j = 0; j < EPRE; j++) key[j] = j < cnt0 ? pk_key(E[j]) : 0u;
+    const uint64_t t = (uint64_t)kth_largest<EPRE>(key, kp) << 32;
+    fl_e = t > fl_e ? t : fl_e;
+    look();
+    more = __ballot(x > 0) != 0;
+    incl = wave_incl_scan(c);
+    M = (int)rdl((uint32_t)incl, 63);
+  }
+  int from = EPRE;  // the first entry of group 0's sub-records not yet in the list
+  if (M > SURV) {   // (ties at the bound: read again below, where the list is cut as it fills)
+    from = 0;
+    x = cnt0;
+    M = 0;
+  } else {
+    int pos = incl - c;
+    uint64_t* const spare = &F.srt[lane];  // non-survivors write here: no exec-mask branches
+#pragma unroll
+    for (int j = 0; j < EPRE; j++) {
+      uint64_t* const dst = ok[j] ? &F.list[pos] : spare;
+      *dst = E[j];
+      pos += ok[j] ? 1 : 0;
+    }
+  }
+  // The list's entries at or above its K'-th largest key, and the floor there.
+  auto trim = [&]() __attribute__((always_inline)) {
+    wave_lds_sync();
+    uint64_t v[SURV / 64];
+    uint32_t key[SURV / 64];
+#pragma unroll
+    for (int r = 0; r < SURV / 64; r++) {
+      v[r] = r * 64 + lane < M ? F.list[r * 64 + lane] : 0ull;
+      key[r] = pk_key(v[r]);
+    }
+    const uint64_t t = (uint64_t)kth_largest<SURV / 64>(key, kp) << 32;
+    fl_e = t > fl_e ? t : fl_e;
+    wave_lds_sync();  // every lane has read the list
+    M = 0;
+#pragma unroll
+    for (int r = 0; r < SURV / 64; r++) {
+      const uint64_t b = __ballot(v[r] != 0ull && v[r] >= fl_e);  // (an entry is never 0)
+      if (v[r] != 0ull && v[r] >= fl_e) F.list[M + lanes_below(b)] = v[r];
+      M += __popcll(b);
+    }
+    wave_lds_sync();
+  };
+#pragma unroll 1
+  for (int g = 0; g < G; g++) {
+    if (g > 0) {  // groups past the first: nothing preloaded
+      const int s = g * 64 + lane;
+      const uint64_t h4 = ld_sub<LOC>(&rowrec[4 * nsp + min(s, nsp - 1)]);  // (clamped, not guarded)
+      x = s < nsub ? (int)min((uint32_t)h4, (uint32_t)CAPW) : 0;
+      from = 0;
+    }
+    if (!__ballot(x > 0)) continue;
+    const int inc = wave_incl_scan(x);
+    const int total = (int)rdl((uint32_t)inc, 63);
+    wave_lds_sync();
+    F.pref[lane] = inc;
+    wave_lds_sync();
+#pragma unroll 1
+    for (int base = 0; base < total; base += 256) {
+      uint64_t e[4];
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        const int t = base + u * 64 + lane;
+        int s = 0;  // sub-records of the group wholly before entry t
+#pragma unroll
+        for (int st = 32; st > 0; st >>= 1) s += F.pref[s + st - 1] <= t ? st : 0;
+        const int j = from + t - (s > 0 ? F.pref[s - 1] : 0);
+        // (clamped inside the sub-record, not guarded: all four in flight)
+        e[u] = ld_sub<LOC>(rowrec + (int64_t)(SHDR + min(max(j, 0), CAPW - 1)) * nsp + g * 64 + s);
+      }
+#pragma unroll 1
+      for (int u = 0; u < 4; u++) {
+        const uint64_t v = u == 0 ? e[0] : u == 1 ? e[1] : u == 2 ? e[2] : e[3];
+        const bool in = base + u * 64 + lane < total;
+        uint64_t b = __ballot(in && v >= fl_e);
+        if (!b) continue;
+        if (M + __popcll(b) > SURV) {  // (M > SURV - 64 >= KSEL >= K' entries)
+          trim();
+          if (M > SURV - 64) {  // ties at the K'-th: its K' best by (logit, id)
+            rank_sort_lds(F.list, F.srt, M);
+            const uint64_t cut = F.srt[kp - 1];
+            fl_e = cut > fl_e ? cut : fl_e;
+#pragma unroll
+            for (int r = 0; r < KSEL / 64; r++)
+              if (r * 64 + lane < kp) F.list[r * 64 + lane] = F.srt[r * 64 + lane];
+            wave_lds_sync();
+            M = kp;
+          }
+          b = __ballot(in && v >= fl_e);
+        }
+        if (in && v >= fl_e) F.list[M + lanes_below(b)] = v;
+        M += __popcll(b);
+      }
+    }
+  }
+  // (the sort that follows counts, for each entry, all the others: 5 us at
+  // 256 of them, where this takes under 1 us)
+  if (M > 64 && M > kp) trim();
+  return M;
+}
+
+// ---------------------------------------------------------------------------
 // Row finalize, common case: at most 64 sub-records (one per lane), K' <= 64,
-// at most SURV survivors, and no boundary
-// tie that needs the id-ordered row scan.  Returns false (having written
+// and no boundary tie that needs the id-ordered row scan.  Returns false (having written
 // nothing) when the row is outside that case; the general finalizer then
 // does the row.  Same arithmetic, in the same order, as the general path.
 template <bool HAS_MASK, bool WANT_LSE, bool LOC>
@@ -1466,9 +1658,12 @@ XS_DEV bool fin_fast(const Args& a, const Cfg& cfg, int row, int nsub, const uin
     M = (int)rdl((uint32_t)incl, 63);
   }
   // entries past the preloaded ones (a sub-record holding more than EPRE); in
-  // a sorted sub-record (flag 4) they end at the first one below the floor
+  // a sorted sub-record (flag 4) they end at the first one below the floor.
+  // Many of them in one sub-record, or more survivors than the list holds:
+  // the general path's gather_survivors.
   const bool srt = (hf & 4u) != 0;
   int lim = (srt && E[EPRE - 1] < floor_e) ? EPRE : cnt;
+  if (XS_RARE(M > SURV || __ballot(lim > 2 * EPRE))) return false;
 #pragma unroll 1
   for (int j0 = EPRE; __ballot(j0 < lim); j0 += 4) {
     uint64_t e[4];
@@ -1479,7 +1674,7 @@ XS_DEV bool fin_fast(const Args& a, const Cfg& cfg, int row, int nsub, const uin
     for (int u = 0; u < 4; u++) put(e[u], j0 + u < lim && e[u] >= floor_e);
     if (srt && j0 + 3 < lim && e[3] < floor_e) lim = j0;
   }
-  if (M > SURV) return false;
+  if (XS_RARE(M > SURV)) return false;
   F.expt[lane] = et;
   wave_lds_sync();
   // rank by counting the survivors above, LDS broadcast reads
@@ -1795,90 +1990,22 @@ XS_DEV void fin_general(const Args& a, const Cfg cfg, int row, const uint64_t* r
   }
 
   // Gather the survivors (entries at or above the bound) into LDS.
-  uint64_t floor_e = (uint64_t)tau_row << 32;
   int M = 0;
-  auto put = [&](uint64_t e, bool ok) __attribute__((always_inline)) {
-    const uint64_t b = __ballot(ok);
-    if (b) {
-      const int pos = M + lanes_below(b);
-      if (ok && pos < SURV) F.list[pos] = e;
-      M += __popcll(b);
-    }
-  };
-  auto gather_global = [&](int g, int s, int c, bool srt, uint64_t fl_e) __attribute__((always_inline)) {
-    // the c entries of sub-record s (the first EPRE of group 0 preloaded, the
-    // rest read from the workspace); in a sorted sub-record (flag 4) they end
-    // at the first one below the floor
-    int lim = c, j = 0;
-    if (g == 0) {
-#pragma unroll
-      for (int u = 0; u < EPRE; u++) put(E[u], u < lim && E[u] >= fl_e);
-      if (srt && EPRE - 1 < lim && E[EPRE - 1] < fl_e) lim = EPRE;
-      j = EPRE;
-    }
-    for (; __ballot(j < lim); j += 4) {
-      uint64_t e[4];
-#pragma unroll
-      for (int u = 0; u < 4; u++)  // (clamped inside the sub-record, not guarded: all four in flight)
-        e[u] = ld_sub<LOC>(rr + (int64_t)(SHDR + min(j + u, CAPW - 1)) * nsp + s);
-#pragma unroll
-      for (int u = 0; u < 4; u++) put(e[u], j + u < lim && e[u] >= fl_e);
-      if (srt && j + 3 < lim && e[3] < fl_e) lim = j;
-    }
-  };
-  auto gather = [&](uint64_t fl_e) __attribute__((always_inline)) {
-    M = 0;
-#pragma unroll
-    for (int g = 0; g < GMAX; g++) {
-      const int s = g * 64 + lane;
-      if (g < G) {
-        const uint64_t h3 = hdr(g, 3), h4 = hdr(g, 4);
-        gather_global(g, s, has(g) ? (int)min((uint32_t)h4, (uint32_t)CAPW) : 0, ((h3 >> 32) & 4u) != 0, fl_e);
-      }
-    }
-  };
-  if (!cfg.bad) gather(floor_e);
-  if (M > SURV) {
-    // More survivors than one wave sorts (ties at the bound across many
-    // waves): move the floor to the exact K'-th largest entry by bisection
-    // over every entry, then gather again.
-    uint64_t ans = 0;
-    for (int bit = 63; bit >= 0; bit--) {
-      const uint64_t cnd = ans | (1ull << bit);
-      int c = 0;
-#pragma unroll
-      for (int g = 0; g < GMAX; g++) {
-        const int s = g * 64 + lane;
-        const int n = has(g) ? (int)min((uint32_t)hdr(g, 4), (uint32_t)CAPW) : 0;
-        for (int j = 0; j < n; j++) c += ld_sub<LOC>(rr + (int64_t)(SHDR + j) * nsp + s) >= cnd ? 1 : 0;
-      }
-      if (wave_sumi(c) >= kp) ans = cnd;
-    }
-    floor_e = ans;
-    gather(floor_e);
+  if (!cfg.bad) {
+    const uint32_t c0 = has(0) ? (uint32_t)h[4] : 0u;
+    M = gather_survivors<LOC>(rr, nsp, nsub, kp, E, (int)min(c0, (uint32_t)CAPW), ((h[3] >> 32) & 4u) != 0,
+                              (uint64_t)tau_row << 32, F);
   }
   F.expt[lane] = et;
   wave_lds_sync();
 
-  // Sort the survivors (logit desc, id asc); the first K' are the selection:
-  // up to 128 by a bitonic sort in registers, more by rank in LDS.
+  // Sort the survivors (logit desc, id asc); the first K' are the selection.
   const int nsel = min(M, kp);  // == kp unless the row holds fewer finite values
   uint64_t sel[2];
-  uint64_t last_sel;  // the K'-th survivor
-  if (M <= 128) {
-    uint64_t x[2];
+  rank_sort_lds(F.list, F.srt, M);
 #pragma unroll
-    for (int r = 0; r < 2; r++) x[r] = (r * 64 + lane < M) ? F.list[r * 64 + lane] : 0ull;  // entries are > 0
-    wave_sort_desc64<2>(x);
-#pragma unroll
-    for (int r = 0; r < 2; r++) sel[r] = (r * 64 + lane < nsel) ? x[r] : 0ull;
-    last_sel = nsel > 0 ? pick64(x, nsel - 1) : 0ull;
-  } else {
-    rank_sort_lds(F.list, F.srt, min(M, SURV));
-#pragma unroll
-    for (int r = 0; r < 2; r++) sel[r] = (r * 64 + lane < nsel) ? F.srt[r * 64 + lane] : 0ull;
-    last_sel = nsel > 0 ? F.srt[nsel - 1] : 0ull;
-  }
+  for (int r = 0; r < 2; r++) sel[r] = (r * 64 + lane < nsel) ? F.srt[r * 64 + lane] : 0ull;
+  const uint64_t last_sel = nsel > 0 ? F.srt[nsel - 1] : 0ull;  // the K'-th survivor
 
   // Probabilities of the selection and the (p desc, id asc) order; p is
   // non-increasing along the logit order, so only runs of equal p move.
@@ -2041,18 +2168,17 @@ XS_DEV void fin_general(const Args& a, const Cfg cfg, int row, const uint64_t* r
 #pragma unroll
                 for (int u = 0; u < 4; u++)  // (clamped inside the sub-record, not guarded)
                   e[u] = ld_sub<LOC>(rr + (int64_t)(SHDR + min(j + u, CAPW - 1)) * nsp + s);
-                uint32_t hb = 0;  // bit u: entry j + u ties
+                uint32_t hb = 0;  // bit u: entry j + u lies in the band
 #pragma unroll
                 for (int u = 0; u < 4; u++) {
-                  const float x = keyf(pk_key(e[u]));
-                  const float d = dv(x);
-                  if (j + u < lim && d >= x_lo && d <= x_hi && exact_p(x, cfg, m_s, S, T) == Pk) hb |= 1u << u;
+                  const float d = dv(keyf(pk_key(e[u])));
+                  if (j + u < lim && d >= x_lo && d <= x_hi) hb |= 1u << u;
                 }
                 if (srt && j + 3 < lim && dv(keyf(pk_key(e[3]))) < x_lo) lim = j;  // the rest lie below
-                while (__ballot(hb != 0u)) {
+                while (__ballot(hb != 0u)) {  // (one copy of the exact exp: code size)
                   const int u = hb ? (int)__builtin_ctz(hb) : 0;
                   const uint64_t eu = u == 0 ? e[0] : u == 1 ? e[1] : u == 2 ? e[2] : e[3];
-                  push(hb != 0u, pk_id(eu));
+                  push(hb != 0u && exact_p(keyf(pk_key(eu)), cfg, m_s, S, T) == Pk, pk_id(eu));
                   hb &= hb - 1u;
                 }
               }
@@ -2088,7 +2214,7 @@ XS_DEV void fin_general(const Args& a, const Cfg cfg, int row, const uint64_t* r
                   v[j] = make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);
                   if (id0 < enc) v[j] = reinterpret_cast<const float4*>(rowp)[id0 >> 2];
                 }
-                uint32_t hb = 0u;  // bit 4j + e: element e of slot j0 + j ties
+                uint32_t hb = 0u;  // bit 4j + e: element e of slot j0 + j lies in the band
 #pragma unroll
                 for (int j = 0; j < 4; j++) {
                   const int id0 = (s0 + j0 + j) * SLOT + 4 * (w * 64 + lane);
@@ -2099,12 +2225,15 @@ XS_DEV void fin_general(const Args& a, const Cfg cfg, int row, const uint64_t* r
                     bool hit = id < enc;
                     if (HAS_MASK && hit && !((mrow[id >> 5] >> (id & 31)) & 1u)) hit = false;
                     const float d = dv(xv[e]);
-                    if (hit && d >= x_lo && d <= x_hi && exact_p(xv[e], cfg, m_s, S, T) == Pk) hb |= 1u << (4 * j + e);
+                    if (hit && d >= x_lo && d <= x_hi) hb |= 1u << (4 * j + e);
                   }
                 }
                 while (__ballot(hb != 0u)) {
                   const int t = hb ? (int)__builtin_ctz(hb) : 0;
-                  push(hb != 0u, (uint32_t)((s0 + j0 + (t >> 2)) * SLOT + 4 * (w * 64 + lane) + (t & 3)));
+                  const float4 vt = t < 4 ? v[0] : t < 8 ? v[1] : t < 12 ? v[2] : v[3];
+                  const float xt = (t & 2) ? ((t & 1) ? vt.w : vt.z) : ((t & 1) ? vt.y : vt.x);
+                  push(hb != 0u && exact_p(xt, cfg, m_s, S, T) == Pk,
+                       (uint32_t)((s0 + j0 + (t >> 2)) * SLOT + 4 * (w * 64 + lane) + (t & 3)));
                   hb &= hb - 1u;
                 }
               }
@@ -2155,25 +2284,24 @@ XS_DEV void fin_general(const Args& a, const Cfg cfg, int row, const uint64_t* r
               }
             }
           }
-          bool hit[4];
-          int c = 0;
+          uint32_t hb = 0u, hits = 0u;  // bit e: element e lies in the band; ties
 #pragma unroll
           for (int e = 0; e < 4; e++) {
-            const int id = 4 * f + e;
-            const float x = xv[e];
-            hit[e] = false;
-            if (id < enc) {
-              const float sx = cfg.scale ? x * cfg.inv : x;
-              const float d = sx - m_s;
-              if (d >= x_lo && d <= x_hi) hit[e] = exact_p(x, cfg, m_s, S, T) == Pk;
-            }
-            c += hit[e];
+            const float d = dv(xv[e]);
+            if (4 * f + e < enc && d >= x_lo && d <= x_hi) hb |= 1u << e;
           }
+          while (__ballot(hb != 0u)) {
+            const int e = hb ? (int)__builtin_ctz(hb) : 0;
+            const float x = e == 0 ? xv[0] : e == 1 ? xv[1] : e == 2 ? xv[2] : xv[3];
+            if (hb != 0u && exact_p(x, cfg, m_s, S, T) == Pk) hits |= 1u << e;
+            hb &= hb - 1u;
+          }
+          const int c = (int)__popc(hits);
           const int incl = wave_incl_scan(c);
           int pos = incl - c;
 #pragma unroll
           for (int e = 0; e < 4; e++)
-            if (hit[e]) {
+            if ((hits >> e) & 1u) {
               if (pos < need) F.psel[have + pos] = ((uint64_t)__float_as_uint(Pk + 0.0f) << 32) | (uint64_t)(0xFFFFFFFFu - (uint32_t)(4 * f + e));
               pos++;
             }
@@ -3071,18 +3199,21 @@ XS_DEV float ser_local(const Args& a, const Cfg& cfg, int row, float m_s, SerLoc
 // After the finalizing wave's finalize_row: when it left a controlled row
 // unsettled (F.need_ser), the wave sums the row's serial denominator
 // (ser_local) and finalizes the row again with it, which settles it by
-// construction.  Rows sent here are counted.
+// construction.  Rows sent here are counted.  (fin_general takes every row;
+// a second copy of fin_fast would only add to the kernel's code, and a loop
+// around one copy of both keeps values live across ser_local: 43 registers
+// spilled.)
 template <bool HAS_MASK, bool WANT_LSE, bool HAS_CTL, bool LOC>
 XS_DEV void ser_fallback(const Args& a, const Cfg& cfg, int row, const uint64_t* rowrec, int nsp, int nsub,
                          const float* rowp, const uint32_t* mrow, TailLds& Tl) {
   wave_lds_sync();  // lane 0 wrote the verdict
-  if (!Tl.fin.need_ser) return;
+  if (!XS_RARE(Tl.fin.need_ser)) return;
   const float m_s = Tl.fin.ser_ms;
   wave_lds_sync();  // read before ser_local reuses the memory
   const float S_ser = ser_local<HAS_MASK, HAS_CTL>(a, cfg, row, m_s, Tl.ser);
   if (lane_id() == 0 && a.ser_count) atomicAdd(a.ser_count, 1u);
   // The record's address and stride pass through an empty asm statement, so
-  // the compiler forms this finalize_row's addresses afresh instead of
+  // the compiler forms this finalization's addresses afresh instead of
   // keeping the first one's live across it (18 such registers spilled to
   // scratch in the masked and controlled kernels).
   // (both made uniform first, so the scalar-register constraint always holds)
@@ -3092,7 +3223,12 @@ XS_DEV void ser_fallback(const Args& a, const Cfg& cfg, int row, const uint64_t*
       (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)ra));
   int np = __builtin_amdgcn_readfirstlane(nsp);
   asm volatile("" : "+s"(rr), "+s"(np));
-  finalize_row<HAS_MASK, WANT_LSE, HAS_CTL, LOC>(a, cfg, row, rr, np, nsub, rowp, mrow, Tl.fin, S_ser);
+  uint64_t h[NHW], E[EPRE];
+  load_heads<WANT_LSE, LOC>(rr, np, nsub, h, E);
+  CtlRow cr{};
+  if (HAS_CTL) cr = a.ctl_row[row];
+  if (lane_id() == 0) Tl.fin.need_ser = 0;
+  fin_general<HAS_MASK, WANT_LSE, HAS_CTL, LOC>(a, cfg, row, rr, np, nsub, rowp, mrow, cr, h, E, Tl.fin, S_ser);
 }
 
 // The row's arrival ticket counts its workgroups (bits 0-7; a row has at most
@@ -3307,7 +3443,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4, 8))) v
     const float ms = mr * inv_e;
     const bool redo = ms > c_s + 40.0f || !(__builtin_fabsf(c_s) < 0x1p20f);
     bool exact_off = false;
-    if (__ballot(redo)) {
+    if (XS_RARE(__ballot(redo))) {
       const float cn = redo ? ms : c_s;
       float s2 = 0.0f;
 #pragma unroll
@@ -3519,7 +3655,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4, 8))) v
   int cnt = 0;
   bool ovf = false;
   uint64_t* const stg = Tl.stage[wave];
-  const float tf = (tk <= KEY_NEG_INF) ? -__FLT_MAX__ : keyf(tk);  // the filter's floor
+  float tf = (tk <= KEY_NEG_INF) ? -__FLT_MAX__ : keyf(tk);  // the filter's floor
   if (!cfg.bad) {
     // every slot's ballot first, so the branches below test values already in
     // scalar registers instead of waiting on each compare
@@ -3543,10 +3679,9 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4, 8))) v
         }
       }
     }
-    if (cnt > CAPW) {  // the exact re-scan writes its entries straight to the sub-record
+    if (XS_RARE(cnt > CAPW)) {  // staged again at a higher floor, or written straight to the sub-record
       const ChunkCtl cc{pl, pc0, phi, ctl_pull, ctl_force, ctl_pval, ctl_fval};
-      cnt = wave_overflow<HAS_MASK, HAS_CTL, LOC>(rowp, mrow, s0, ns, enc, sub, nsp, kp, tk, cc);
-      ovf = true;
+      cnt = wave_overflow<HAS_MASK, HAS_CTL, LOC>(rowp, mrow, s0, ns, enc, sub, nsp, kp, stg, tf, ovf, cc);
     }
   }
   // More entries than the finalizer preloads (EPRE), at most 64: stored in
