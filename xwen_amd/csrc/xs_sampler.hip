@@ -31,7 +31,7 @@
 //   verify       for a speculative block, the last row finalizer of a
 //                sequence runs accept_drafts over the sequence's rows.
 //   controls     a call with sparse controls first runs control_kernel (one
-//                workgroup per row), which turns the row's bans and biases into
+//                workgroup per chunk of a row), which turns the row's bans and biases into
 //                a sorted list of final values, and keeps the pulled and the
 //                forced values, for the chunk pass to apply.
 //
@@ -1576,10 +1576,10 @@ XS_DEV int gather_survivors(const uint64_t* rowrec, int nsp, int nsub, int kp, c
 // and no boundary tie that needs the id-ordered row scan.  Returns false (having written
 // nothing) when the row is outside that case; the general finalizer then
 // does the row.  Same arithmetic, in the same order, as the general path.
-template <bool HAS_MASK, bool WANT_LSE, bool LOC>
-XS_DEV bool fin_fast(const Args& a, const Cfg& cfg, int row, int nsub, const uint64_t (&h)[NHW],
-                     const uint64_t (&E)[EPRE], const uint64_t* rowrec, int nsp, const float* rowp,
-                     FinLds& F, float S_ser) {
+template <bool HAS_MASK, bool WANT_LSE, bool HAS_CTL, bool LOC>
+XS_DEV bool fin_fast(const Args& a, const Cfg& cfg, int row, int nsub, const CtlRow& cr,
+                     const uint64_t (&h)[NHW], const uint64_t (&E)[EPRE], const uint64_t* rowrec, int nsp,
+                     const float* rowp, FinLds& F, float S_ser) {
   const int lane = lane_id();
   const bool live = lane < nsub;
   const bool stoch = !cfg.greedy;
@@ -1605,8 +1605,10 @@ XS_DEV bool fin_fast(const Args& a, const Cfg& cfg, int row, int nsub, const uin
   const double S_d = red_sumd(part);
   const double R_d = WANT_LSE ? red_sumd(rpart) : 0.0;
   const float S = S_ser >= 0.0f ? S_ser : (float)S_d;  // a controlled row's serial sum, when given
+  const bool ctl_on = HAS_CTL && cr.active;
   int st = XS_ROW_OK;
-  if (HAS_MASK && !finite_seen) st = XS_ROW_NO_FINITE;
+  if (ctl_on && cr.status != XS_ROW_OK) st = cr.status;
+  else if ((HAS_MASK || ctl_on) && !finite_seen) st = XS_ROW_NO_FINITE;
   else if (cfg.greedy) st = nan_seen ? XS_ROW_NAN : (m_v == -INFINITY ? XS_ROW_NO_FINITE : XS_ROW_OK);
   else if (nan_seen || __builtin_isinf(m_s)) st = XS_ROW_NAN;
 
@@ -1704,10 +1706,10 @@ XS_DEV bool fin_fast(const Args& a, const Cfg& cfg, int row, int nsub, const uin
   uint64_t pk = 0ull;
   float w = 0.0f;
   int tok = -1;
-  // a masked row not given the serial sum: its token is checked against the
-  // roundings that sum could change (order_settled, draw_settled); with one
-  // finite value the token is that id for every denominator
-  const bool check = HAS_MASK && S_ser < 0.0f && nsel > 1;
+  // a controlled row not given the serial sum: its token is checked against
+  // the roundings that sum could change (order_settled, draw_settled); with
+  // one finite value the token is that id for every denominator
+  const bool check = (HAS_MASK || ctl_on) && S_ser < 0.0f && nsel > 1;
   bool unsettled = false;
   if (stoch && st == XS_ROW_OK) {
     const float vL = nsel > 0 ? keyf(pk_key(rdl64(sel, nsel - 1))) : -INFINITY;
@@ -2581,8 +2583,8 @@ XS_DEV void finalize_heads(const Args& a, const Cfg& cfg, int row, const uint64_
   CtlRow cr{};
   if (HAS_CTL) cr = a.ctl_row[row];
   if (lane_id() == 0) F.need_ser = 0;
-  const bool done = !(HAS_CTL && cr.active) && nsub <= 64 && cfg.kp <= 64 && !cfg.bad && !cfg.big &&
-                    fin_fast<HAS_MASK, WANT_LSE, LOC>(a, cfg, row, nsub, h, E, rowrec, nsp, rowp, F, S_ser);
+  const bool done = nsub <= 64 && cfg.kp <= 64 && !cfg.bad && !cfg.big &&
+                    fin_fast<HAS_MASK, WANT_LSE, HAS_CTL, LOC>(a, cfg, row, nsub, cr, h, E, rowrec, nsp, rowp, F, S_ser);
   if (!done) fin_general<HAS_MASK, WANT_LSE, HAS_CTL, LOC>(a, cfg, row, rowrec, nsp, nsub, rowp, mrow, cr, h, E, F, S_ser);
 }
 
@@ -3316,6 +3318,12 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4, 8))) v
     ctl_fval = cr.force_val;
   }
   const int pc0 = pc;  // the chunk's first patch
+  // The next 64 patches, one per lane, read in one load: a patch read from
+  // memory where it applies cost its round trip each (16 rows of 300 entries,
+  // 19 a chunk: sample_kernel 29 -> 22 us, with fin_fast for controlled rows).
+  uint64_t pw = 0ull;
+  int pb = pc;  // the patch lane 0 holds
+  if (HAS_CTL && pc < phi) pw = pl[min(pc + lane, phi - 1)];
 
   // Online reduction, one float4 at a time, branch-free.  The softmax partial
   // is summed in the reference's scaled domain, s = v * inv rounded to f32 as
@@ -3378,7 +3386,11 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4, 8))) v
         } else {
           // this slot's patches: the next ones in the sorted list
           while (pc < phi) {
-            const uint64_t pe = pl[pc];
+            if (pc - pb == 64) {
+              pb = pc;
+              pw = pl[min(pc + lane, phi - 1)];
+            }
+            const uint64_t pe = rdl64(pw, pc - pb);
             const int off = (int)(uint32_t)(pe >> 32) - sb;
             if (off >= SLOT) break;
             if ((off >> 2) == tid) {
@@ -4267,182 +4279,270 @@ __global__ __launch_bounds__(BLOCK) void serial_kernel(Args a) {
 }
 
 // ---------------------------------------------------------------------------
-// Sparse controls (apply_control, sampler.rs:433-490): one workgroup per row,
-// launched before sample_kernel when a call carries controls.  The row's bans
-// and biases become its patch list: every distinct listed id < enc with its
-// value after the mask, the bans (sampler.rs:450-454) and then the biases in
-// list order (:455-459).  A pull needs the row max after those (:460-470): the
-// workgroup reads the row once for it, and only for a finite target, and keeps
-// the target's new value.  A force keeps the target's final value (:471-482).
-// sample_kernel overwrites exactly these elements before anything reads them.
+// Sparse controls (apply_control, sampler.rs:433-490), launched before
+// sample_kernel when a call carries controls: one workgroup per chunk of a
+// row.  Chunk 0's workgroup makes the row's patch list from its bans and
+// biases: every distinct listed id < enc with its value after the mask, the
+// bans (sampler.rs:450-454) and then the biases in list order (:455-459).  A
+// pull needs the row max after those (:460-470): every chunk's workgroup
+// takes the max over its unlisted ids (a bitmap of the listed ones in LDS),
+// and the row's last to arrive (an arrival ticket, slots 4 and 5 of the row's
+// ticket line) forms the target's new value.  The other chunks' workgroups of
+// a row without a pull return at once.  A force keeps the target's final value
+// (:471-482).  sample_kernel overwrites exactly these elements before anything
+// reads them.
+//
+// Latency-bound.  One workgroup reading a pulled row alone, a float4 a thread
+// at a time with a search of the list per value, took 276 us for 16 rows of
+// 248,320 ids with lists of 300; a chunk per workgroup, all its loads in
+// flight, 17 us.
+constexpr int CTL_RANK = 512;  // lists sorted by counting (two entries a thread; above it, bitonic)
 template <bool HAS_MASK>
 __global__ __launch_bounds__(BLOCK) void control_kernel(Args a) {
   __shared__ uint64_t lkeys[CTL_MAX];  // (id << 32 | list position), sorted (lists of CTL_MAX or fewer)
   __shared__ uint64_t lpl[CTL_MAX];    // the patch list (idem)
   __shared__ SortLds B;                // the radix sort's counters (longer lists)
+  __shared__ uint32_t listed[SPC * SLOT / 32];  // this chunk's listed ids
   __shared__ int s4[NWAVE];
   __shared__ float wmax[NWAVE];
-  const int row = blockIdx.x, tid = threadIdx.x, lane = lane_id(), wave = wave_id();
+  const int nc = a.n_chunks;
+  const int row = blockIdx.x / nc, chunk = blockIdx.x - row * nc;
+  const int tid = threadIdx.x, lane = lane_id(), wave = wave_id();
   const xs_row_control c = a.controls[row];
-  const int enc = (int)a.enc, nc = a.n_chunks;
+  const int enc = (int)a.enc;
   const float* rowp = a.logits + (int64_t)row * a.ld;
   const uint32_t* mrow = HAS_MASK ? a.allowed + (int64_t)row * a.allowed_ld : nullptr;
   int32_t* cb = a.ctl_chunk + (int64_t)row * (nc + 1);
   uint64_t* patch = a.patch + (int64_t)row * a.ctl_cap;
-  auto allowed = [&](int id) __attribute__((always_inline)) {
-    return !HAS_MASK || ((mrow[id >> 5] >> (id & 31)) & 1u);
-  };
   const bool active = c.n_ban != 0 || c.n_bias != 0 || c.has_pull != 0 || c.has_force != 0;
   const int64_t n64 = (int64_t)c.n_ban + (int64_t)c.n_bias;
   int status = XS_ROW_OK;
   if (c.n_ban < 0 || c.n_bias < 0 || c.ban_off < 0 || c.bias_off < 0 || n64 > a.ctl_cap ||
       (n64 > 0 && !a.ctl_ids) || (c.n_bias > 0 && !a.ctl_delta))
     status = XS_ROW_BAD_PARAM;
-  if (!active || status != XS_ROW_OK) {
+  const bool good = active && status == XS_ROW_OK;
+  const bool pulls = good && c.has_pull && c.pull_id < (uint32_t)enc;
+  if (chunk != 0 && !pulls) return;
+  if (!good) {
     for (int i = tid; i <= nc; i += BLOCK) cb[i] = 0;
     if (tid == 0) a.ctl_row[row] = CtlRow{active ? 1 : 0, status, 0, -1, 0.0f, -1, 0.0f, 0};
     return;
   }
-
-  // Sort the listed ids, each tagged with its list position (bans first):
-  // a list of CTL_MAX or fewer in LDS (bitonic), a longer one in the
-  // context's sort buffers (the stable LSD radix sort of the whole-row path,
-  // by ~id descending, which keeps equal ids in list order); the patch list
-  // then goes straight to the row's patch array.
   const int n = (int)n64;
-  const bool lds = n <= CTL_MAX;
-  uint64_t* const gk = lds ? nullptr : a.ctl_keys + (int64_t)row * 2 * a.ctl_cap;
-  uint64_t* const pl = lds ? lpl : patch;
-  if (lds) {
-    int np2 = 1;
-    while (np2 < n) np2 <<= 1;
-    for (int i = tid; i < np2; i += BLOCK) {
-      uint64_t k = ~0ull;
-      if (i < n) {
-        const uint32_t id = i < c.n_ban ? a.ctl_ids[c.ban_off + i] : a.ctl_ids[c.bias_off + (i - c.n_ban)];
-        k = ((uint64_t)id << 32) | (uint32_t)i;
-      }
-      lkeys[i] = k;
-    }
+  auto list_id = [&](int i) __attribute__((always_inline)) -> uint32_t {
+    return i < c.n_ban ? a.ctl_ids[c.ban_off + i] : a.ctl_ids[c.bias_off + (i - c.n_ban)];
+  };
+  // the row max after the bans and biases, as an order-preserving key
+  // (f32::max folds skip NaN; so does every `>` test here)
+  uint32_t* const rmax = reinterpret_cast<uint32_t*>(&a.row_ticket[row * TSTRIDE + 4]);
+  auto block_best = [&](float best) __attribute__((always_inline)) {  // (all threads; a barrier inside)
+    best = wave_maxf(best);
+    if (lane == 0) wmax[wave] = best;
     __syncthreads();
-    for (int size = 2; size <= np2; size <<= 1) {  // bitonic, ascending
-      for (int stride = size >> 1; stride > 0; stride >>= 1) {
-        for (int i = tid; i < np2 / 2; i += BLOCK) {
-          const int lo = 2 * i - (i & (stride - 1)), hi = lo + stride;
-          const bool asc = (lo & size) == 0;
-          const uint64_t x = lkeys[lo], y = lkeys[hi];
-          if ((x > y) == asc) {
-            lkeys[lo] = y;
-            lkeys[hi] = x;
-          }
-        }
-        __syncthreads();
-      }
-    }
-  } else {
-    for (int i = tid; i < n; i += BLOCK) {
-      const uint32_t id = i < c.n_ban ? a.ctl_ids[c.ban_off + i] : a.ctl_ids[c.bias_off + (i - c.n_ban)];
-      gk[i] = ((uint64_t)(0xFFFFFFFFu - id) << 32) | (uint32_t)i;
-    }
-    __syncthreads();
-    radix_sort_desc(gk, gk + a.ctl_cap, n, B);  // (every pass ends in a barrier)
-  }
-  auto keys = [&](int i) __attribute__((always_inline)) -> uint64_t {  // (id << 32 | list position)
-    if (lds) return lkeys[i];
-    const uint64_t k = gk[i];
-    return ((uint64_t)(0xFFFFFFFFu - (uint32_t)(k >> 32)) << 32) | (uint32_t)k;
-  };
-
-  // One patch per distinct id < enc: the run of its entries holds its bans
-  // (lower positions) and then its biases in list order.
-  const int seg = (n + BLOCK - 1) / BLOCK;
-  const int b0 = min(n, tid * seg), b1 = min(n, b0 + seg);
-  auto starts = [&](int i) __attribute__((always_inline)) {
-    const uint32_t id = (uint32_t)(keys(i) >> 32);
-    return id < (uint32_t)enc && (i == 0 || (uint32_t)(keys(i - 1) >> 32) != id);
-  };
-  int cnt = 0;
-  for (int i = b0; i < b1; i++) cnt += starts(i) ? 1 : 0;
-  int total;
-  int p = block_excl_scan(cnt, s4, &total);
-  for (int i = b0; i < b1; i++) {
-    if (!starts(i)) continue;
-    const uint32_t id = (uint32_t)(keys(i) >> 32);
-    float x = allowed((int)id) ? rowp[id] : -INFINITY;
-    for (int j = i; j < n && (uint32_t)(keys(j) >> 32) == id; j++) {
-      const int o = (int)(uint32_t)keys(j);
-      if (o < c.n_ban) x = -INFINITY;
-      else x = x + a.ctl_delta[c.bias_off + (o - c.n_ban)];
-    }
-    pl[p++] = ((uint64_t)id << 32) | __float_as_uint(x);
-  }
-  __syncthreads();
-  auto lower = [&](uint32_t v) __attribute__((always_inline)) {  // first patch with id >= v
-    int lo = 0, hi = total;
-    while (lo < hi) {
-      const int mid = (lo + hi) >> 1;
-      if ((uint32_t)(pl[mid] >> 32) < v) lo = mid + 1;
-      else hi = mid;
-    }
-    return lo;
-  };
-  auto patched = [&](int id) __attribute__((always_inline)) {
-    const int q = lower((uint32_t)id);
-    return q < total && (uint32_t)(pl[q] >> 32) == (uint32_t)id;
-  };
-  if (lds)
-    for (int i = tid; i < total; i += BLOCK) patch[i] = pl[i];
-  for (int i = tid; i <= nc; i += BLOCK) cb[i] = (i == nc) ? total : lower((uint32_t)(i * SPC * SLOT));
-
-  // pull: the max M over the row after the bans and biases (f32::max folds
-  // skip NaN; so does every `>` test here), then v += alpha * max(0, M - v)
-  int pull_id = -1;
-  float pull_val = 0.0f;
-  if (c.has_pull && c.pull_id < (uint32_t)enc) {
-    const int t = (int)c.pull_id;
-    const float vt = patched(t) ? __uint_as_float((uint32_t)pl[lower((uint32_t)t)])
-                                : (allowed(t) ? rowp[t] : -INFINITY);
-    if (__builtin_isfinite(vt)) {
-      float best = -INFINITY;
-      const v4f* r4 = reinterpret_cast<const v4f*>(rowp);
-      for (int f = tid; 4 * f < enc; f += BLOCK) {
-        const v4f q = r4[f];
+    if (tid == 0) {
+      float m = wmax[0];
 #pragma unroll
-        for (int e = 0; e < 4; e++) {
-          const int id = 4 * f + e;
-          const float x = q4(q, e);
-          if (id < enc && x > best && allowed(id) && !patched(id)) best = x;
+      for (int w = 1; w < NWAVE; w++) m = wmax[w] > m ? wmax[w] : m;
+      __hip_atomic_fetch_max(rmax, fkey(m), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+  };
+  if (pulls) {
+    const v4f* r4 = reinterpret_cast<const v4f*>(rowp);
+    const int fmax = (enc - 1) >> 2, s0 = chunk * SPC;
+    v4f q[SPC];
+    uint32_t mw[SPC];
+#pragma unroll
+    for (int j = 0; j < SPC; j++) {  // (clamped, not guarded: all in flight)
+      const int f = min((s0 + j) * BLOCK + tid, fmax);
+      q[j] = r4[f];
+      if (HAS_MASK) mw[j] = mrow[f >> 3];
+    }
+    for (int i = tid; i < SPC * SLOT / 32; i += BLOCK) listed[i] = 0u;
+    __syncthreads();
+    for (int i = tid; i < n; i += BLOCK) {
+      const uint32_t id = list_id(i);
+      if (id / (uint32_t)(SPC * SLOT) == (uint32_t)chunk)
+        atomicOr(&listed[(id % (uint32_t)(SPC * SLOT)) >> 5], 1u << (id & 31u));
+    }
+    __syncthreads();
+    float best = -INFINITY;
+#pragma unroll
+    for (int j = 0; j < SPC; j++) {
+      const int id0 = ((s0 + j) * BLOCK + tid) * 4;  // this float4's first id (past enc: none of it counts)
+      const int sh = id0 & 31;
+      uint32_t skip = listed[(j * SLOT + 4 * tid) >> 5] >> sh;
+      if (HAS_MASK) skip |= ~(mw[j] >> sh);
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const float x = q4(q[j], e);
+        if (id0 + e < enc && x > best && !((skip >> e) & 1u)) best = x;
+      }
+    }
+    block_best(best);
+  }
+
+  if (chunk == 0) {
+    // Sort the listed ids, each tagged with its list position (bans first):
+    // a list of CTL_MAX or fewer in LDS (short ones by counting each entry's
+    // smaller ones, longer ones bitonic: at 512 entries 1 us against 3, at
+    // 2,048 14 against 8), a longer one in the context's sort buffers (the
+    // stable LSD radix sort of the whole-row path, by ~id descending, which
+    // keeps equal ids in list order); the patch list then goes straight to
+    // the row's patch array.
+    const bool lds = n <= CTL_MAX;
+    uint64_t* const gk = lds ? nullptr : a.ctl_keys + (int64_t)row * 2 * a.ctl_cap;
+    uint64_t* const pl = lds ? lpl : patch;
+    if (n <= CTL_RANK) {
+      uint64_t k[CTL_RANK / BLOCK];
+      int rk[CTL_RANK / BLOCK];
+#pragma unroll
+      for (int r = 0; r < CTL_RANK / BLOCK; r++) {
+        const int i = r * BLOCK + tid;
+        k[r] = i < n ? ((uint64_t)list_id(i) << 32) | (uint32_t)i : ~0ull;
+        lpl[i] = k[r];
+        rk[r] = 0;
+      }
+      __syncthreads();
+#pragma unroll 8
+      for (int j = 0; j < n; j++) {
+        const uint64_t y = lpl[j];
+#pragma unroll
+        for (int r = 0; r < CTL_RANK / BLOCK; r++) rk[r] += y < k[r] ? 1 : 0;
+      }
+#pragma unroll
+      for (int r = 0; r < CTL_RANK / BLOCK; r++)
+        if (r * BLOCK + tid < n) lkeys[rk[r]] = k[r];
+      __syncthreads();
+    } else if (lds) {
+      int np2 = 1;
+      while (np2 < n) np2 <<= 1;
+      for (int i = tid; i < np2; i += BLOCK) lkeys[i] = i < n ? ((uint64_t)list_id(i) << 32) | (uint32_t)i : ~0ull;
+      __syncthreads();
+      for (int size = 2; size <= np2; size <<= 1) {  // bitonic, ascending
+        for (int stride = size >> 1; stride > 0; stride >>= 1) {
+          for (int i = tid; i < np2 / 2; i += BLOCK) {
+            const int lo = 2 * i - (i & (stride - 1)), hi = lo + stride;
+            const bool asc = (lo & size) == 0;
+            const uint64_t x = lkeys[lo], y = lkeys[hi];
+            if ((x > y) == asc) {
+              lkeys[lo] = y;
+              lkeys[hi] = x;
+            }
+          }
+          __syncthreads();
         }
       }
-      for (int i = tid; i < total; i += BLOCK) {
-        const float v = __uint_as_float((uint32_t)pl[i]);
-        if (v > best) best = v;
-      }
-      best = wave_maxf(best);
-      if (lane == 0) wmax[wave] = best;
-      __syncthreads();
-      float M = wmax[0];
-      for (int w = 1; w < NWAVE; w++) M = wmax[w] > M ? wmax[w] : M;
-      pull_val = vt + c.pull_alpha * fmaxf(M - vt, 0.0f);
-      pull_id = t;
-    }
-  }
-  // force: the target keeps its final value if finite, else 0
-  int force_id = -1;
-  float force_val = 0.0f;
-  if (c.has_force) {
-    if (c.force_id >= (uint32_t)enc) {
-      status = XS_ROW_FORCE_OOR;
     } else {
-      const int t = (int)c.force_id;
-      const float v = t == pull_id ? pull_val
-                                   : (patched(t) ? __uint_as_float((uint32_t)pl[lower((uint32_t)t)])
-                                                 : (allowed(t) ? rowp[t] : -INFINITY));
-      force_val = __builtin_isfinite(v) ? v : 0.0f;
-      force_id = t;
+      for (int i = tid; i < n; i += BLOCK) gk[i] = ((uint64_t)(0xFFFFFFFFu - list_id(i)) << 32) | (uint32_t)i;
+      __syncthreads();
+      radix_sort_desc(gk, gk + a.ctl_cap, n, B);  // (every pass ends in a barrier)
+    }
+    auto keys = [&](int i) __attribute__((always_inline)) -> uint64_t {  // (id << 32 | list position)
+      if (lds) return lkeys[i];
+      const uint64_t k = gk[i];
+      return ((uint64_t)(0xFFFFFFFFu - (uint32_t)(k >> 32)) << 32) | (uint32_t)k;
+    };
+    auto masked_value = [&](int id) __attribute__((always_inline)) {  // (both loads in flight together)
+      const float x = rowp[id];
+      const bool in = !HAS_MASK || ((mrow[id >> 5] >> (id & 31)) & 1u);
+      return in ? x : -INFINITY;
+    };
+
+    // One patch per distinct id < enc: the run of its entries holds its bans
+    // (lower positions) and then its biases in list order.
+    const int seg = (n + BLOCK - 1) / BLOCK;
+    const int b0 = min(n, tid * seg), b1 = min(n, b0 + seg);
+    auto starts = [&](int i) __attribute__((always_inline)) {
+      const uint32_t id = (uint32_t)(keys(i) >> 32);
+      return id < (uint32_t)enc && (i == 0 || (uint32_t)(keys(i - 1) >> 32) != id);
+    };
+    int cnt = 0;
+    for (int i = b0; i < b1; i++) cnt += starts(i) ? 1 : 0;
+    int total;
+    int p = block_excl_scan(cnt, s4, &total);
+    float best = -INFINITY;  // of this thread's patches
+    for (int i = b0; i < b1; i++) {
+      if (!starts(i)) continue;
+      const uint32_t id = (uint32_t)(keys(i) >> 32);
+      float x = masked_value((int)id);
+      for (int j = i; j < n && (uint32_t)(keys(j) >> 32) == id; j++) {
+        const int o = (int)(uint32_t)keys(j);
+        if (o < c.n_ban) x = -INFINITY;
+        else x = x + a.ctl_delta[c.bias_off + (o - c.n_ban)];
+      }
+      best = x > best ? x : best;
+      pl[p++] = ((uint64_t)id << 32) | __float_as_uint(x);
+    }
+    __syncthreads();
+    auto lower = [&](uint32_t v) __attribute__((always_inline)) {  // first patch with id >= v
+      int lo = 0, hi = total;
+      while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        if ((uint32_t)(pl[mid] >> 32) < v) lo = mid + 1;
+        else hi = mid;
+      }
+      return lo;
+    };
+    auto value = [&](int id) __attribute__((always_inline)) {  // after the mask, the bans and the biases
+      const int q = lower((uint32_t)id);
+      return q < total && (uint32_t)(pl[q] >> 32) == (uint32_t)id ? __uint_as_float((uint32_t)pl[q])
+                                                                  : masked_value(id);
+    };
+    if (lds)
+      for (int i = tid; i < total; i += BLOCK) patch[i] = pl[i];
+    for (int i = tid; i <= nc; i += BLOCK) cb[i] = (i == nc) ? total : lower((uint32_t)(i * SPC * SLOT));
+    if (pulls) block_best(best);
+
+    // The pull's target and its value before the pull, and only if that is
+    // finite; the force's target, which keeps its final value if finite, else
+    // 0.  Both are completed below when the row's max is known.
+    if (tid == 0) {
+      CtlRow cr{1, status, total, -1, 0.0f, -1, 0.0f, 0};
+      if (pulls) {
+        const float vt = value((int)c.pull_id);
+        if (__builtin_isfinite(vt)) {
+          cr.pull_id = (int)c.pull_id;
+          cr.pull_val = vt;
+        }
+      }
+      if (c.has_force) {
+        if (c.force_id >= (uint32_t)enc) {
+          cr.status = XS_ROW_FORCE_OOR;
+        } else {
+          const float v = value((int)c.force_id);
+          cr.force_val = __builtin_isfinite(v) ? v : 0.0f;
+          cr.force_id = (int)c.force_id;
+        }
+      }
+      // (agent scope: the row's last workgroup may run on another XCD)
+      uint64_t w[sizeof(CtlRow) / 8];
+      __builtin_memcpy(w, &cr, sizeof(cr));
+      uint64_t* const dst = reinterpret_cast<uint64_t*>(&a.ctl_row[row]);
+#pragma unroll
+      for (int i = 0; i < (int)(sizeof(CtlRow) / 8); i++) st_agent(&dst[i], w[i]);
     }
   }
-  if (tid == 0) a.ctl_row[row] = CtlRow{1, status, total, pull_id, pull_val, force_id, force_val, 0};
+  if (!pulls) return;
+
+  // pull: v += alpha * max(0, M - v) with the row's max M
+  if (tid == 0) {
+    drain();  // this workgroup's max (and chunk 0's CtlRow) are performed
+    int32_t* const tk = &a.row_ticket[row * TSTRIDE + 5];
+    if (__hip_atomic_fetch_add(tk, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == nc - 1) {
+      const float M = keyf((uint32_t)ld_agent(reinterpret_cast<const int32_t*>(rmax)));
+      st_agent(tk, 0);
+      st_agent(reinterpret_cast<int32_t*>(rmax), 0);
+      CtlRow* const cr = &a.ctl_row[row];
+      const int pull_id = ld_agent(&cr->pull_id);
+      if (pull_id >= 0) {
+        const float vt = __int_as_float(ld_agent(reinterpret_cast<const int32_t*>(&cr->pull_val)));
+        const float pv = vt + c.pull_alpha * fmaxf(M - vt, 0.0f);
+        st_agent(reinterpret_cast<int32_t*>(&cr->pull_val), __float_as_int(pv));
+        if (ld_agent(&cr->force_id) == pull_id)
+          st_agent(reinterpret_cast<int32_t*>(&cr->force_val), __float_as_int(__builtin_isfinite(pv) ? pv : 0.0f));
+      }
+    }
+  }
 }
 
 // Fills every row's status with one data error (a call-level condition such as
@@ -5335,7 +5435,7 @@ void launch2(xs_context* ctx, xs::Args& a, int64_t rows, dim3 g1, dim3 gs, const
   // finalizers then overlap the later rows' streaming inside one launch (C5:
   // 75 us in one launch, 91 us split; C4: 57.2 us in one, 55.4 us split).
   a.split = ((g1.x > (unsigned)(4 * ctx->n_cu) && !S && !order) || ctx->xcd_test == 1) ? 1 : 0;
-  if (C) hipLaunchKernelGGL((xs::control_kernel<M>), dim3((unsigned)rows), dim3(xs::BLOCK), 0, ctx->stream, a);
+  if (C) hipLaunchKernelGGL((xs::control_kernel<M>), g1, dim3(xs::BLOCK), 0, ctx->stream, a);
   // (a call of fewer rows than XCDs drops its row order: its rows all start
   // at once, and outputs do not depend on the order)
   if (order && loc) {
