@@ -500,6 +500,31 @@ class Sampler:
         k_max = _lib.K_MAX if opts.top_k <= _lib.K_MAX else min(int(opts.top_k), encodable)
         self.ctx = Context(max_rows, encodable, k_max=max(k_max, _lib.K_MAX), device=device)
         self.device = f"cuda:{device}"
+        self._bufs = self._buffers(max_rows)
+        self._params = None
+
+    @staticmethod
+    def _buffers(rows):
+        """What a call of up to `rows` rows exchanges with the host: the
+        uniforms it draws from and the tokens and statuses it leaves, in pinned
+        memory that the kernels read and write in place, so that a call makes
+        no copies (4 rows: 89 us a call with three uploads, two allocations and
+        two read-backs, 34 without).  A call ends with its stream's
+        synchronize, so the next one may reuse them."""
+        torch = _torch()
+        host = torch.empty((3, rows), dtype=torch.int32, pin_memory=True)
+        view = host.numpy()
+        return {"rows": rows, "host": host, "u": view[0].view(np.float32), "token": view[1], "status": view[2]}
+
+    def _row_params(self, rows, device):
+        """xs_row_params for every row of a call, kept on the device while the
+        options stay the same."""
+        key = (self.opts.temperature, self.opts.top_k, self.opts.top_p, device)
+        if self._params is None or self._params[0] != key or self._params[1] < rows:
+            n = max(rows, self.ctx.max_rows)
+            self._params = (key, n, params_tensor(self.opts.temperature, self.opts.top_k, self.opts.top_p,
+                                                  n, device))
+        return self._params[2]
 
     def encodable(self) -> int:
         return self.encodable_
@@ -532,20 +557,28 @@ class Sampler:
             logits = padded
         if uniforms is None:
             uniforms = self.next_uniforms(rows)
-        u = torch.as_tensor(np.asarray(uniforms, np.float32), device=logits.device)
-        p = params_tensor(self.opts.temperature, self.opts.top_k, self.opts.top_p, rows,
-                          logits.device)
+        b = self._bufs
+        if rows > b["rows"]:
+            b = self._bufs = self._buffers(rows)
+        u = np.asarray(uniforms, np.float32).reshape(-1)
+        if u.size < rows:
+            raise ValueError(f"{rows} rows need as many uniforms, got {u.size}")
+        b["u"][:rows] = u[:rows]
+        p = self._row_params(rows, logits.device)
         allowed = None if ctl is None else ctl.allowed
         controls = None
         if ctl is not None and ctl.has_sparse():
             controls = controls_tensor([ctl] * rows, logits.device)
+        stream = torch.cuda.current_stream(self.ctx.device)
         self.ctx.bind_current_stream()
-        out = sample_batch(self.ctx, logits, p, u, enc=self.encodable_, width=width,
-                           allowed=allowed, controls=controls)
-        st = out.status.cpu().numpy()
+        host = b["host"]
+        sample_batch(self.ctx, logits, p, host[0], enc=self.encodable_, width=width, allowed=allowed,
+                     controls=controls, out=Draws(token=host[1], status=host[2]))
+        stream.synchronize()
+        st = b["status"][:rows]
         if st.any():
-            raise SampleError(st)
-        return out.token.cpu().numpy().astype(np.int64)
+            raise SampleError(st.copy())
+        return b["token"][:rows].astype(np.int64)
 
     def sample(self, logits, uniforms=None):
         return self.sample_controlled(logits, None, uniforms)
