@@ -420,7 +420,7 @@ struct Args {
   double* class_mass;
   double* probs;
   int64_t probs_ld;
-  uint64_t* score_part;  // [rows, n_chunks, XS_CLASS_MAX] the chunks' class sums (f64 bits)
+  uint64_t* score_part;  // [rows, score_parts, XS_CLASS_MAX] the parts' class sums (f64 bits)
   // verify walk (span == 0: plain batch)
   int32_t span;
   const int32_t* drafts;
@@ -3856,58 +3856,53 @@ __global__ __launch_bounds__(BLOCK) void finalize_kernel(Args a) {
 // ---------------------------------------------------------------------------
 // score_kernel: the scoring reads of held rows, launched after sample_kernel
 // has written each row's lse (held_row, generate.rs:1905-1933).  Grid: rows x
-// n_chunks, the chunks of sample_kernel.  Each workgroup forms, for the ids of
-// its chunk, p = exp(f64(v) - lse) -- the reference's last_probs term
+// score_parts, a part being SCORE_SPP slots.  Each workgroup forms, for the
+// ids of its part, p = exp(f64(v) - lse) -- the reference's last_probs term
 // (generate.rs:1893-1899), written out when `probs` is asked for -- and adds
 // the p of each class's ids, as escape_mass sums last_probs over its classes
 // (batch.rs:1638-1662).  The row's last workgroup to arrive (an arrival
-// ticket, slot 3 of the row's ticket line) adds the chunks' class sums in
-// chunk order.  Chunk 0's workgroup also reads the scored ids:
-// f64(v[id]) - lse, and an id outside [0, enc) fails the row as
-// last_logprobs_for does (generate.rs:1871-1883).  A row whose held_row
-// failed (NaN lse) keeps its status; its scores are NaN.
-__global__ __launch_bounds__(BLOCK) void score_kernel(Args a) {
+// ticket, slot 3 of the row's ticket line) adds the parts' class sums, lane by
+// lane and then across the lanes: the same order whichever comes last.  Part
+// 0's workgroup also reads the scored ids: f64(v[id]) - lse, and an id outside
+// [0, enc) fails the row as last_logprobs_for does (generate.rs:1871-1883); a
+// call that asks for nothing else launches that part alone.  A row whose
+// held_row failed (NaN lse) keeps its status; its scores are NaN.
+//
+// Bound by latency at the few rows a scored field has: a part is four slots,
+// all its loads in flight, and the last workgroup reads the parts' sums at
+// once.  One workgroup per 16 slots, a slot's load waited for at a time and
+// the sums read one after another, took 33 us for 16 rows of 248,320 ids with
+// two classes; now 17 us, of which the f64 exps are about 5.
+constexpr int SCORE_SPP = 4;
+constexpr int score_parts(int nslots) { return (nslots + SCORE_SPP - 1) / SCORE_SPP; }
+__global__ __launch_bounds__(BLOCK) void score_kernel(Args a, int np) {
   __shared__ double expt[64];
   __shared__ double part[NWAVE][XS_CLASS_MAX];
   __shared__ int32_t last;
   const int tid = threadIdx.x, lane = lane_id(), wave = wave_id();
-  const int nc = a.n_chunks;
-  const int row = blockIdx.x / nc, chunk = blockIdx.x - row * nc;
+  const int row = blockIdx.x / np, pt = blockIdx.x - row * np;
   const int enc = (int)a.enc;
   const int ncl = a.class_masks ? a.n_class : 0;
+  const bool sums = a.probs || ncl > 0;
+  const float* rowp = a.logits + (int64_t)row * a.ld;
+  const int fmax = (enc - 1) >> 2, s0 = pt * SCORE_SPP;
+  float4 q[SCORE_SPP];
+  uint32_t w[XS_CLASS_MAX][SCORE_SPP];
+  if (sums) {
+#pragma unroll
+    for (int j = 0; j < SCORE_SPP; j++)  // (clamped to the row's last float4, not guarded: all in flight)
+      q[j] = reinterpret_cast<const float4*>(rowp)[min((s0 + j) * BLOCK + tid, fmax)];
+#pragma unroll
+    for (int c = 0; c < XS_CLASS_MAX; c++) {
+      const uint32_t* cm = a.class_masks + ((int64_t)row * a.n_class + c) * a.class_ld;
+#pragma unroll
+      for (int j = 0; j < SCORE_SPP; j++) w[c][j] = c < ncl ? cm[min((s0 + j) * BLOCK + tid, fmax) >> 3] : 0u;
+    }
+  }
   if (tid < 64) expt[tid] = (&kExpT[0][0])[tid];
   const double lse = a.row_lse[row];
   const bool ok = !__builtin_isnan(lse);
-  const float* rowp = a.logits + (int64_t)row * a.ld;
-  __syncthreads();
-  double acc[XS_CLASS_MAX];
-#pragma unroll
-  for (int c = 0; c < XS_CLASS_MAX; c++) acc[c] = 0.0;
-  const int s0 = chunk * SPC;
-  const int ns = min(SPC, a.nslots - s0);
-  for (int j = 0; j < ns; j++) {
-    const int id0 = ((s0 + j) * BLOCK + tid) * 4;
-    if (id0 < enc) {  // (the float4 lies inside the row: ld % 4 == 0 and id0 < enc <= ld)
-      const float4 v = reinterpret_cast<const float4*>(rowp)[id0 >> 2];
-      const float xv[4] = {v.x, v.y, v.z, v.w};
-      uint32_t w[XS_CLASS_MAX];
-#pragma unroll
-      for (int c = 0; c < XS_CLASS_MAX; c++)
-        w[c] = c < ncl ? a.class_masks[((int64_t)row * a.n_class + c) * a.class_ld + (id0 >> 5)] : 0u;
-#pragma unroll
-      for (int e = 0; e < 4; e++) {
-        const int id = id0 + e;
-        if (id < enc) {
-          const double p = ok ? exp_f64((double)xv[e] - lse, expt) : __builtin_nan("");
-          if (a.probs) a.probs[(int64_t)row * a.probs_ld + id] = p;
-#pragma unroll
-          for (int c = 0; c < XS_CLASS_MAX; c++)
-            if (c < ncl && ((w[c] >> (id & 31)) & 1u)) acc[c] += p;
-        }
-      }
-    }
-  }
-  if (chunk == 0 && a.score_ids) {
+  if (pt == 0 && a.score_ids) {
     bool oor = false;
     for (int i = tid; i < a.n_score; i += BLOCK) {
       const int id = a.score_ids[(int64_t)row * a.score_ld + i];
@@ -3920,8 +3915,29 @@ __global__ __launch_bounds__(BLOCK) void score_kernel(Args a) {
       a.token[row] = -1;
     }
   }
+  if (!sums) return;
+  __syncthreads();  // expt
+  double acc[XS_CLASS_MAX];
+#pragma unroll
+  for (int c = 0; c < XS_CLASS_MAX; c++) acc[c] = 0.0;
+#pragma unroll
+  for (int j = 0; j < SCORE_SPP; j++) {
+    const int id0 = ((s0 + j) * BLOCK + tid) * 4;
+    const float xv[4] = {q[j].x, q[j].y, q[j].z, q[j].w};
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      const int id = id0 + e;
+      if (id < enc) {
+        const double p = ok ? exp_f64((double)xv[e] - lse, expt) : __builtin_nan("");
+        if (a.probs) a.probs[(int64_t)row * a.probs_ld + id] = p;
+#pragma unroll
+        for (int c = 0; c < XS_CLASS_MAX; c++)
+          if (c < ncl && ((w[c][j] >> (id & 31)) & 1u)) acc[c] += p;
+      }
+    }
+  }
   if (ncl == 0) return;
-  // the chunk's class sums: waves in order, then the row's chunks in order
+  // the part's class sums, waves in order
 #pragma unroll
   for (int c = 0; c < XS_CLASS_MAX; c++) {
     if (c < ncl) {
@@ -3930,25 +3946,29 @@ __global__ __launch_bounds__(BLOCK) void score_kernel(Args a) {
     }
   }
   __syncthreads();
-  uint64_t* const prow = a.score_part + (int64_t)row * nc * XS_CLASS_MAX;
+  uint64_t* const prow = a.score_part + (int64_t)row * np * XS_CLASS_MAX;
   if (tid < ncl) {
     double t = 0.0;
 #pragma unroll
-    for (int w = 0; w < NWAVE; w++) t += part[w][tid];
-    st_agent(&prow[chunk * XS_CLASS_MAX + tid], (uint64_t)__double_as_longlong(t));
+    for (int v = 0; v < NWAVE; v++) t += part[v][tid];
+    st_agent(&prow[pt * XS_CLASS_MAX + tid], (uint64_t)__double_as_longlong(t));
   }
   drain();
   __syncthreads();
   if (tid == 0) {
     const int t = __hip_atomic_fetch_add(&a.row_ticket[row * TSTRIDE + 3], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    last = (t == nc - 1) ? 1 : 0;
-    if (t == nc - 1) st_agent(&a.row_ticket[row * TSTRIDE + 3], 0);
+    last = (t == np - 1) ? 1 : 0;
+    if (t == np - 1) st_agent(&a.row_ticket[row * TSTRIDE + 3], 0);
   }
   __syncthreads();
-  if (!last || tid >= ncl) return;
-  double m = 0.0;
-  for (int k = 0; k < nc; k++) m += __longlong_as_double((long long)ld_agent(&prow[k * XS_CLASS_MAX + tid]));
-  a.class_mass[(int64_t)row * a.n_class + tid] = m;
+  if (!last) return;
+  // wave v adds classes v and v + NWAVE
+  for (int c = wave; c < ncl; c += NWAVE) {
+    double m = 0.0;
+    for (int k = lane; k < np; k += 64) m += __longlong_as_double((long long)ld_agent(&prow[k * XS_CLASS_MAX + c]));
+    m = wave_sumd(m);
+    if (lane == 0) a.class_mass[(int64_t)row * a.n_class + c] = m;
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -5389,7 +5409,7 @@ struct xs_context {
   uint32_t* ser_count;  // [1] rows the finalizers summed serially themselves (ser_local), or null
   int32_t ser_force;    // test hook: every checked row takes that fallback
   double* lse_ws;       // [max_rows] held_row lse of calls that score without taking row_lse
-  uint64_t* score_part; // [max_rows, max_chunks, XS_CLASS_MAX] score_kernel's chunk class sums
+  uint64_t* score_part; // [max_rows, score_parts, XS_CLASS_MAX] score_kernel's class sums by part
 };
 
 namespace {
@@ -5578,7 +5598,7 @@ int xs_create_ex(int device, int64_t max_rows, int64_t vocab, int32_t k_max, int
   ok = ok && hipMalloc((void**)&c->ser_e, max_rows * xs::SER_NB * (xs::SEG / 2) * sizeof(uint64_t)) == hipSuccess;
   ok = ok && hipMalloc((void**)&c->ser_count, sizeof(uint32_t)) == hipSuccess;
   ok = ok && hipMalloc((void**)&c->lse_ws, max_rows * sizeof(double)) == hipSuccess;
-  ok = ok && hipMalloc((void**)&c->score_part, (size_t)max_rows * mc * XS_CLASS_MAX * sizeof(uint64_t)) == hipSuccess;
+  ok = ok && hipMalloc((void**)&c->score_part, (size_t)max_rows * xs::score_parts(mc * xs::SPC) * XS_CLASS_MAX * sizeof(uint64_t)) == hipSuccess;
   ok = ok && hipMemset(c->ser_count, 0, sizeof(uint32_t)) == hipSuccess;
   if (k_max > XS_K_MAX) {  // top_k past the streaming selection: the whole-row path's buffers
     ok = ok && hipMalloc((void**)&c->big, (size_t)max_rows * 2 * vocab * sizeof(uint64_t)) == hipSuccess;
@@ -5752,7 +5772,9 @@ int sample_impl(xs_context* ctx, const xs_sample_args* in, bool clear_tickets) {
   // fails the caller's row)
   a.token = in->token;
   a.status = in->status;
-  hipLaunchKernelGGL(xs::score_kernel, dim3((unsigned)(in->rows * a.n_chunks)), dim3(xs::BLOCK), 0, ctx->stream, a);
+  const int np = (a.probs || a.n_class > 0) ? xs::score_parts(a.nslots) : 1;
+  if (in->rows * (int64_t)np > 0x7FFFFFFF) return XS_ERR_CAPACITY;
+  hipLaunchKernelGGL(xs::score_kernel, dim3((unsigned)(in->rows * np)), dim3(xs::BLOCK), 0, ctx->stream, a, np);
   return hipGetLastError() == hipSuccess ? XS_OK : XS_ERR_HIP;
 }
 }  // namespace
