@@ -1313,9 +1313,18 @@ XS_DEV void held_fold(const Args& a, int row, const float* rowp, const uint64_t*
 //    with |r| <= (k + j + 2) 2^-24 (each p, the k-term sum, the division, j
 //    additions); x = rn(u T_w) is within (k + keep + 3) 2^-24 of u times its
 //    exact total; twice each (S and S'), plus the p's subnormal ulps.
-// A row that fails is summed serially by its finalizing wave (ser_local)
-// and finalized again with S'.  The order part (order_settled) runs as soon
-// as the selection's e are known, the margins (draw_settled) after the draw.
+// The order part (order_settled) runs as soon as the selection's e are known,
+// the margins (draw_settled) after the draw.  Two weaker conditions are enough
+// where those fail:
+//  - entries that some D rounds to one p are ordered by id among themselves:
+//    a run of them whose ids ascend along the logit order keeps its order for
+//    every D, and another one matters to a call that takes tokens only when
+//    the drawn entry lies in it (order_settled gives those positions);
+//  - the draw by itself and the cuts on either side of top_p (draw_refined).
+// A row that fails those too is summed serially by its finalizing wave
+// (ser_local) and finalized again with S'.  That costs a row of 248,320 ids
+// 1.3 ms; of 2,560 random masked rows at top_k 100 it took 51 without the
+// weaker conditions and 6 with them, of 960 at top_k 50 2 and 0.
 template <int R>
 XS_DEV float at_lane(const float (&v)[R], int i) {  // element i of a list held R per lane (i uniform)
   float out = 0.0f;
@@ -1362,9 +1371,12 @@ XS_DEV float below_selection(const uint64_t* rowrec, int nsp, int nsub, const ui
   return wave_maxf(best);
 }
 
+// (sel: the selection in logit order.  amb: the positions, by bit, whose entry
+// may change with the denominator, for a call that takes tokens only; with
+// candidates any such position fails.)
 template <int R>
-XS_DEV bool order_settled(const float (&ee)[R], int nsel, int kp, int k, bool full, float e_below, float S,
-                          float dthr, bool cands) {
+XS_DEV bool order_settled(const float (&ee)[R], const uint64_t (&sel)[R], int nsel, int kp, int k, bool full,
+                          float e_below, float S, float dthr, bool cands, uint64_t (&amb)[R]) {
   const int lane = lane_id();
   const float thr = S * dthr;  // 2^-148 D for every D the serial sum can take (f32: the constants carry 1 %)
   const float NEG = 0x1p-65f;
@@ -1375,6 +1387,7 @@ XS_DEV bool order_settled(const float (&ee)[R], int nsel, int kp, int k, bool fu
   bool bad = false;
 #pragma unroll
   for (int r = 0; r < R; r++) {  // consecutive selected entries i, i + 1
+    amb[r] = 0ull;
     const float first_next = (r + 1 < R) ? rdlf(ee[r + 1 < R ? r + 1 : r], 0) : 0.0f;
     const float en = lane == 63 ? first_next : __shfl(ee[r], (lane + 1) & 63);
     const int i = r * 64 + lane;
@@ -1391,7 +1404,47 @@ XS_DEV bool order_settled(const float (&ee)[R], int nsel, int kp, int k, bool fu
     const float below = all_sel ? 0.0f : e_below;
     if (e1 == eL && (cands || e1 >= NEG) && !(below < eL && robust(eL, below))) ubad = true;
   }
-  return __ballot(bad) == 0 && !ubad;
+  if (XS_RARE(__ballot(bad) != 0)) {
+    // the runs of entries whose p may be equal (link i: entries i and i + 1),
+    // from the first: one with a pair that is not robust and a pair whose ids
+    // descend may be reordered
+    bool run_open = false, run_desc = false;
+    int start = 0;
+#pragma unroll 1
+    for (int i = 0; i < nsel; i++) {
+      bool link = false;
+      if (i + 1 < nsel) {
+        const float ea = at_lane(ee, i), eb = at_lane(ee, i + 1);
+        const bool rob = robust(ea, eb);
+        link = ea == eb || !rob;
+        if (link) {
+          run_open = run_open || (!rob && (cands || ea >= NEG));
+          run_desc = run_desc || pk_id(pick64(sel, i)) > pk_id(pick64(sel, i + 1));
+        }
+      }
+      if (!link) {
+        // (a run that reaches the last selected entry may go on below it)
+        if (i == nsel - 1 && !all_sel && !full) {
+          const float eL = at_lane(ee, i);
+          run_desc = run_desc || !(e_below < eL && robust(eL, e_below));
+        }
+        if (run_open && run_desc) {
+#pragma unroll
+          for (int q = 0; q < R; q++) {
+            const int lo = max(start - 64 * q, 0), hi = min(i - 64 * q, 63);  // bits lo..hi of word q
+            if (lo <= hi) amb[q] |= (~0ull >> (63 - hi)) & (~0ull << lo);
+          }
+        }
+        run_open = run_desc = false;
+        start = i + 1;
+      }
+    }
+    if (cands) {
+#pragma unroll
+      for (int q = 0; q < R; q++) ubad = ubad || amb[q] != 0ull;
+    }
+  }
+  return !ubad;
 }
 template <int R>
 XS_DEV bool draw_settled(const float (&c)[R], float tot, float x, int idx, int keep, int k, bool cut_found,
@@ -1418,6 +1471,65 @@ XS_DEV bool draw_settled(const float (&c)[R], float tot, float x, int idx, int k
     if (j == idx && j < keep - 1 && !(cj - x > m + mt)) bad = true;  // x < cum_idx (at keep - 1: the total)
   }
   return __ballot(bad) == 0;
+}
+
+// draw_settled's decisions again where its margins fail, for a call that takes
+// tokens only.
+//
+// The draw by itself: with w_i = kappa e_i (1 + t_i), |t_i| <= 2 2^-24 (p and
+// its division), the prefix c_j = sum of its w_i + d_j, |d_j| <= 2^-24 j c_j,
+// and x = rn(u c_m), m = keep - 1, the difference x - c_j misses kappa (u E_m -
+// E_j) by (u - 1) and u times the errors on either side of j:
+//   2^-24 [2 ((1 - u) c_j + u (c_m - c_j)) + (1 - u) j c_j + u (m - j) c_m + u c_m]
+// since c_m contains c_j's own errors; kappa scales both sides alike for every
+// D.  Twice that (S and S'), with 2 % to spare, and the p's subnormal ulps.
+//
+// The cut: where the margin around top_p leaves two choices of keep (the entry
+// before or after), the draw must give the same index, by the same margins,
+// with either.  wn: the weight of entry keep (the first cut), 0 when there is
+// none.  A cut that leaves three choices fails.
+template <int R>
+XS_DEV bool draw_refined(const float (&c)[R], float tot, float wn, float u, int idx, int keep, int k,
+                         bool cut_found, bool renorm, float S, float top_p) {
+  const int lane = lane_id();
+  const float uu = 0x1p-23f * 1.02f;
+  const float sl = (float)(2 * k + 8) * 0x1p-148f * S + 0x1p-50f;
+  auto draw = [&](int kept, float total) __attribute__((always_inline)) {
+    const float x = u * total + 0.0f;
+    bool bad = false;
+    int n = 0;
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+      const int j = r * 64 + lane;
+      const float cj = c[r];
+      n += (int)__popcll(__ballot(j < k - 1 && (j < kept - 1 ? cj : total) <= x));
+      // (one more u total: the total of another cut is formed by one addition here)
+      const float B = 2.0f * ((1.0f - u) * cj + u * (total - cj)) + (1.0f - u) * (float)j * cj +
+                      u * (float)(kept - 1 - j) * total + 2.0f * u * total;
+      const float m = uu * B + sl;
+      if (j == idx - 1 && !(x - cj > m)) bad = true;
+      if (j == idx && j < kept - 1 && !(cj - x > m)) bad = true;
+    }
+    return n == idx && __ballot(bad) == 0;
+  };
+  auto mc = [&](int j, float cj) __attribute__((always_inline)) { return uu * (float)(k + j + 4) * cj + sl; };
+  if (!draw(keep, tot)) return false;
+  if (!renorm) return true;
+  if (!cut_found) {  // (reached at k - 1 or not at all: all k are kept)
+    return k < 2 || top_p - at_lane(c, k - 2) > mc(k - 2, at_lane(c, k - 2));
+  }
+  if (!(tot - top_p > mc(keep - 1, tot)) && keep < k) {  // the cut may come one entry later
+    const float t2 = tot + wn;
+    if (!(t2 - top_p > mc(keep, t2)) || !draw(keep + 1, t2)) return false;
+  }
+  if (keep >= 2) {
+    const float c1 = at_lane(c, keep - 2);
+    if (!(top_p - c1 > mc(keep - 2, c1))) {  // or one entry earlier
+      if (keep >= 3 && !(top_p - at_lane(c, keep - 3) > mc(keep - 3, at_lane(c, keep - 3)))) return false;
+      if (!draw(keep - 1, c1)) return false;
+    }
+  }
+  return true;
 }
 
 // ---------------------------------------------------------------------------
@@ -1711,6 +1823,7 @@ XS_DEV bool fin_fast(const Args& a, const Cfg& cfg, int row, int nsub, const Ctl
   // one finite value the token is that id for every denominator
   const bool check = (HAS_MASK || ctl_on) && S_ser < 0.0f && nsel > 1;
   bool unsettled = false;
+  uint64_t amb[1] = {0ull};
   if (stoch && st == XS_ROW_OK) {
     const float vL = nsel > 0 ? keyf(pk_key(rdl64(sel, nsel - 1))) : -INFINITY;
     const bool need_below = !cfg.full && vL != -INFINITY;
@@ -1741,7 +1854,8 @@ XS_DEV bool fin_fast(const Args& a, const Cfg& cfg, int row, int nsub, const Ctl
       // row's actual next logit rather than next_below(vL)
       if (!cfg.full && nsel == kp && nsel > k && rdlf(ee, k - 1) == rdlf(ee, nsel - 1))
         ebelow = exact_e(below_selection<LOC>(rowrec, nsp, nsub, E, vL), cfg, m_s, T);
-      unsettled = !order_settled<1>(ea, nsel, kp, k, cfg.full, ebelow, S, cfg.dthr, want_cands);
+      const uint64_t sa[1] = {sel};
+      unsettled = !order_settled<1>(ea, sa, nsel, kp, k, cfg.full, ebelow, S, cfg.dthr, want_cands, amb);
     }
     // (p desc, id asc): p is non-increasing along the logit order, so only
     // runs of equal p can be out of order
@@ -1819,8 +1933,13 @@ XS_DEV bool fin_fast(const Args& a, const Cfg& cfg, int row, int nsub, const Ctl
         tok = (int)pk_id(rdl64(pk, idx));
         if (check) {
           const float ca[1] = {c};
-          unsettled = unsettled || cfg.force ||
-                      !draw_settled<1>(ca, tot, x_draw, idx, keep, k, found, renorm, S, cfg.top_p);
+          bool ok = draw_settled<1>(ca, tot, x_draw, idx, keep, k, found, renorm, S, cfg.top_p);
+          if (XS_RARE(!ok && !want_cands)) {
+            const float pn = __uint_as_float((uint32_t)(rdl64(pk, min(keep, 63)) >> 32));
+            ok = draw_refined<1>(ca, tot, keep < k ? __fdiv_rn(pn, sumc) : 0.0f, u_row, idx, keep, k, found, renorm,
+                                 S, cfg.top_p);
+          }
+          unsettled = unsettled || cfg.force || !ok || ((amb[0] >> idx) & 1ull);
         }
       }
     }
@@ -2027,6 +2146,7 @@ XS_DEV void fin_general(const Args& a, const Cfg cfg, int row, const uint64_t* r
   // one finite value the token is that id for every denominator
   const bool check = (HAS_MASK || ctl_on) && S_ser < 0.0f && nsel > 1;
   bool unsettled = false;
+  uint64_t amb[2] = {0ull, 0ull};
   bool lazy_order = false;  // the (p desc, id asc) repair left to the draw
   if (stoch && st == XS_ROW_OK && !cfg.big) {
     const bool need_below = !cfg.full && vL != -INFINITY;
@@ -2062,7 +2182,7 @@ XS_DEV void fin_general(const Args& a, const Cfg cfg, int row, const uint64_t* r
       // row's actual next logit rather than next_below(vL)
       if (!cfg.full && nsel == kp && nsel > k && at_lane(ee, k - 1) == at_lane(ee, nsel - 1))
         ebelow = exact_e(below_selection<LOC>(rr, nsp, nsub, E, vL), cfg, m_s, T);
-      unsettled = !order_settled<2>(ee, nsel, kp, k, cfg.full, ebelow, S, cfg.dthr, want_cands);
+      unsettled = !order_settled<2>(ee, sel, nsel, kp, k, cfg.full, ebelow, S, cfg.dthr, want_cands, amb);
     }
     bool bad = false;
     const uint64_t n0 = shfl64(pk[0], (lane + 1) & 63);
@@ -2438,9 +2558,15 @@ XS_DEV void fin_general(const Args& a, const Cfg cfg, int row, const uint64_t* r
               tok = (int)y;
             }
           }
-          if (check)
-            unsettled = unsettled || cfg.force ||
-                        !draw_settled<2>(c, tot, x_draw, idx, keep, k, found, renorm, S, cfg.top_p);
+          if (check) {
+            bool ok = draw_settled<2>(c, tot, x_draw, idx, keep, k, found, renorm, S, cfg.top_p);
+            if (XS_RARE(!ok && !want_cands)) {
+              const float pn = __uint_as_float((uint32_t)(pick64(pk, min(keep, 127)) >> 32));
+              ok = draw_refined<2>(c, tot, keep < k ? __fdiv_rn(pn, sumc) : 0.0f, u_row, idx, keep, k, found, renorm,
+                                   S, cfg.top_p);
+            }
+            unsettled = unsettled || cfg.force || !ok || ((amb[idx >> 6] >> (idx & 63)) & 1ull);
+          }
         }
       }
     }
@@ -3872,7 +3998,7 @@ __global__ __launch_bounds__(BLOCK) void finalize_kernel(Args a) {
 // all its loads in flight, and the last workgroup reads the parts' sums at
 // once.  One workgroup per 16 slots, a slot's load waited for at a time and
 // the sums read one after another, took 33 us for 16 rows of 248,320 ids with
-// two classes; now 17 us, of which the f64 exps are about 5.
+// two classes; now 17 us.
 constexpr int SCORE_SPP = 4;
 constexpr int score_parts(int nslots) { return (nslots + SCORE_SPP - 1) / SCORE_SPP; }
 __global__ __launch_bounds__(BLOCK) void score_kernel(Args a, int np) {
