@@ -456,10 +456,12 @@ struct Args {
   uint64_t* big;     // [rows, 2, big_ld]: the whole-row sort's buffers (contexts with k_max > XS_K_MAX)
   int64_t big_ld;
   struct BigRow* big_state;  // [rows]: what the finalizer leaves for the whole-row kernels
-  uint32_t* big_hist;        // [rows, big_hld]: per-tile digit counts (then first positions) of a sort pass
+  uint32_t* big_hist;        // [rows, big_hld]: per-tile digit counts (then first positions) of a sort pass,
+                             // then big_tiles_max counts of the tiles' entries
   int64_t big_hld;
   int32_t* big_ticket;       // [rows * TSTRIDE]: the sort passes' arrival tickets, zero between kernels
   int32_t big_tiles;         // tiles of BTILE ids per row
+  int32_t big_tiles_max;     // and of the context's widest row
   int32_t big_nblk;          // chain blocks per row past the first CHEAD terms
   int32_t big_cut;           // tokens only, enc <= 2^20: rows at top_k >= enc sort only p >= 2^-26
   // the serial denominator (serial_kernel), on calls with a mask or controls:
@@ -4859,10 +4861,12 @@ XS_DEV uint64_t digit_peers(uint32_t d, bool valid) {
   return m;
 }
 XS_DEV uint64_t lanes_below() { return (1ull << lane_id()) - 1ull; }
-// Count this lane's digit once per group of equal digits (the group's lowest lane).
+// Count this lane's digit.  (One LDS add a lane: grouping equal digits first
+// by digit_peers costs some 50 instructions to save the conflicts, which 256
+// digits seldom make, and bound the counting passes: 64 rows of 248,320 ids,
+// big_hist_kernel 24 -> 17 us, big_scatter_kernel 37 -> 33.)
 XS_DEV void count_digit(uint32_t* cnt, uint32_t d, bool valid) {
-  const uint64_t pe = digit_peers(d, valid);
-  if (valid && (pe & lanes_below()) == 0) atomicAdd(&cnt[d], (uint32_t)__popcll(pe));
+  if (valid) atomicAdd(&cnt[d], 1u);
 }
 
 // The row's whole-row state for the kernels below: null when the call does not
@@ -4917,11 +4921,18 @@ XS_DEV void big_counts(const Args& a, int row, int tile, uint32_t c, int32_t* s4
   }
 }
 
+// Per tile of a row, the entries big_key_kernel left for the sort's first pass
+// (after the row's digit counts in big_hist).
+XS_DEV int32_t* big_count(const Args& a, int row) {
+  return reinterpret_cast<int32_t*>(a.big_hist) + (int64_t)(row + 1) * a.big_hld - a.big_tiles_max;
+}
+
 // Grid: rows x big_tiles.  The sort keys of the tile's ids and the first
 // pass's digit counts.
 template <bool HAS_MASK, bool HAS_CTL>
 __global__ __launch_bounds__(BLOCK) void big_key_kernel(Args a) {
-  __shared__ struct { uint2 ent[NWAVE][SPT * 256]; } Kl;  // per wave: (value bits, id) for the exact p
+  __shared__ uint2 ent[BTILE];  // a cut row's ids left for the exact p, in id order: (value bits, id)
+  __shared__ int32_t seg[SPT * NWAVE];  // their counts per slot and wave
   __shared__ double expt[64];
   __shared__ uint32_t hist[RBINS];
   __shared__ int32_t s4[NWAVE];
@@ -4964,8 +4975,10 @@ __global__ __launch_bounds__(BLOCK) void big_key_kernel(Args a) {
   __syncthreads();
   uint64_t* const A = a.big + (int64_t)row * 2 * a.big_ld;
   const int lane = lane_id(), wave = wave_id();
-  int nl = 0;  // this wave's ids left for the exact p (a cut row)
+  uint32_t needs = 0u;  // a cut row: bit 4j + e, element e of slot j is left for the exact p
   const float invS = 1.0f / S;
+  if (cut && tid < SPT * NWAVE) seg[tid] = 0;  // (absent slots)
+  if (cut) __syncthreads();
 #pragma unroll
   for (int j = 0; j < SPT; j++) {
     if (j >= ns) break;  // (uniform)
@@ -4980,19 +4993,18 @@ __global__ __launch_bounds__(BLOCK) void big_key_kernel(Args a) {
     if (ctl_on) ctl_slot(x, sb, tid, pl, pc, phi, cr.pull_id, cr.pull_val, cr.force_id, cr.force_val);
     if (cut) {
       // the plain estimate decides the ids well below the cut; the others go
-      // to the wave's list, for the exact p below with every lane busy
+      // to the tile's list, for the exact p below with every lane busy
+      int c = 0;
 #pragma unroll
       for (int e = 0; e < 4; e++) {
-        const int id = id0 + e;
-        const bool in = id < enc;
         const float sv = cfg.scale ? x[e] * cfg.inv : x[e];
         const float pa = xexp2((sv - m_s) * LOG2E) * invS;
-        const bool need = in && !(pa < PLO);
-        const uint64_t b = __ballot(need);
-        if (need) Kl.ent[wave][nl + lanes_below(b)] = make_uint2(__float_as_uint(x[e]), (uint32_t)id);
-        nl += (int)__popcll(b);
-        if (in && !need) A[id] = ((uint64_t)KSENT << 32) | (uint32_t)id;
+        const bool need = id0 + e < enc && !(pa < PLO);
+        needs |= need ? 1u << (4 * j + e) : 0u;
+        c += (int)__popcll(__ballot(need));
       }
+      q[j] = make_float4(x[0], x[1], x[2], x[3]);
+      if (lane == 0) seg[j * NWAVE + wave] = c;
       continue;
     }
     uint32_t k[4];
@@ -5010,19 +5022,49 @@ __global__ __launch_bounds__(BLOCK) void big_key_kernel(Args a) {
         if (id0 + e < enc) A[id0 + e] = ((uint64_t)k[e] << 32) | (uint32_t)(id0 + e);
     }
   }
+  int n = min(BTILE, enc - tile * BTILE);  // the tile's entries for the sort
   if (cut) {
-    wave_lds_sync();
+    // compacted in id order (slot, then wave, then lane, then element): the
+    // sort's first pass reads these entries only.  With a marked entry per id
+    // instead, that pass and this kernel moved the whole row (64 rows of
+    // 248,320 ids, a quarter of them kept: the pass 96 -> 37 us, this kernel
+    // 81 -> 59)
+    __syncthreads();
+    n = 0;
+    int at[SPT];
+#pragma unroll
+    for (int i = 0; i < SPT * NWAVE; i++) {
+      if (i % NWAVE == wave) at[i / NWAVE] = n;
+      n += seg[i];
+    }
+#pragma unroll
+    for (int j = 0; j < SPT; j++) {
+      const uint32_t nb = (needs >> (4 * j)) & 15u;
+      uint64_t b[4];
+      int pos = at[j];
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        b[e] = __ballot((nb >> e) & 1u);
+        pos += lanes_below(b[e]);
+      }
+      const float x[4] = {q[j].x, q[j].y, q[j].z, q[j].w};
+#pragma unroll
+      for (int e = 0; e < 4; e++)
+        if ((nb >> e) & 1u) ent[pos++] = make_uint2(__float_as_uint(x[e]), (uint32_t)((s0 + j) * SLOT + 4 * tid + e));
+    }
+    __syncthreads();
 #pragma unroll 1
-    for (int b0 = 0; b0 < nl; b0 += 64) {
-      const int i = b0 + lane;
-      const bool v = i < nl;
-      const uint2 it = Kl.ent[wave][v ? i : 0];
+    for (int b0 = 0; b0 < n; b0 += BLOCK) {
+      const int i = b0 + tid;
+      const bool v = i < n;
+      const uint2 it = ent[v ? i : 0];
       uint32_t k = pkey(exact_p(__uint_as_float(it.x), cfg, m_s, S, expt));
       if (k > KCUT) k = KSENT;  // (below the cut after all)
       count_digit(hist, rdigit(k, 0), v && k != KSENT);
-      if (v) A[it.y] = ((uint64_t)k << 32) | it.y;
+      if (v) A[tile * BTILE + i] = ((uint64_t)k << 32) | it.y;
     }
   }
+  if (tid == 0) big_count(a, row)[tile] = n;
   __syncthreads();
   big_counts(a, row, tile, hist[tid], s4, last, a.big_tiles);
 }
@@ -5076,22 +5118,24 @@ __global__ __launch_bounds__(BLOCK) void big_scatter_kernel(Args a, int pass) {
   const int row = blockIdx.x / a.big_tiles, tile = blockIdx.x % a.big_tiles;
   Cfg cfg;
   if (!big_live(a, row, cfg)) return;
-  // the first pass reads every id (in id order, KSENT on those left out),
-  // the others the entries it sorted
+  // the first pass reads what the key kernel left of the tile's ids (in id
+  // order, KSENT on a few left out), the others the entries it sorted; each
+  // wave takes a quarter of them
   if (pass > 0 && tile >= big_sorted_tiles(a, row)) return;
   const int tid = threadIdx.x, lane = lane_id(), wave = wave_id();
-  const int t0 = tile * BTILE, nt = min(BTILE, (pass == 0 ? (int)a.enc : big_sorted(a, row)) - t0);
+  const int t0 = tile * BTILE, nt = pass == 0 ? big_count(a, row)[tile] : min(BTILE, big_sorted(a, row) - t0);
+  const int steps = (nt + BLOCK - 1) / BLOCK;  // (at most EPL)
   uint64_t* const A = a.big + (int64_t)row * 2 * a.big_ld;
   const uint64_t* src = A + ((pass & 1) ? a.big_ld : 0) + t0;
   uint64_t* dst = A + ((pass & 1) ? 0 : a.big_ld);
   const uint32_t first = a.big_hist[(int64_t)row * a.big_hld + (int64_t)tile * RBINS + tid];
-  const int q0 = wave * QW;
+  const int q0 = wave * steps * 64;
   {
     uint64_t e[EPL];  // all of the quarter's loads in flight at once
 #pragma unroll
     for (int s = 0; s < EPL; s++) {
       const int i = q0 + s * 64 + lane;
-      e[s] = i < nt ? src[i] : 0ull;
+      e[s] = s < steps && i < nt ? src[i] : 0ull;
     }
 #pragma unroll
     for (int s = 0; s < EPL; s++) ent[wave][s * 64 + lane] = e[s];
@@ -5101,10 +5145,9 @@ __global__ __launch_bounds__(BLOCK) void big_scatter_kernel(Args a, int pass) {
   for (int i = lane; i < RBINS; i += 64) cnt[wave][i] = 0u;
   wave_lds_sync();
 #pragma unroll 1
-  for (int s = 0; s < EPL; s++) {
+  for (int s = 0; s < steps; s++) {
     const uint32_t key = (uint32_t)(ent[wave][s * 64 + lane] >> 32);
     count_digit(cnt[wave], rdigit(key, pass), q0 + s * 64 + lane < nt && key != KSENT);
-    wave_lds_sync();
   }
   __syncthreads();
   // each wave's first position of every digit (thread t: digit t)
@@ -5118,7 +5161,7 @@ __global__ __launch_bounds__(BLOCK) void big_scatter_kernel(Args a, int pass) {
   __syncthreads();
   // the entries, in order
 #pragma unroll 1
-  for (int s = 0; s < EPL; s++) {
+  for (int s = 0; s < steps; s++) {
     const uint64_t e = ent[wave][s * 64 + lane];
     const bool valid = q0 + s * 64 + lane < nt && (uint32_t)(e >> 32) != KSENT;
     const uint32_t d = rdigit((uint32_t)(e >> 32), pass);
@@ -5545,7 +5588,7 @@ struct xs_context {
   int32_t* seq_ticket;  // [max_rows * TSTRIDE]
   uint64_t* big;        // [max_rows, 2, vocab] whole-row sort buffers (k_max > XS_K_MAX), or null
   xs::BigRow* big_state;  // [max_rows] (with big)
-  uint32_t* big_hist;   // [max_rows, big_tiles_max, RBINS] (with big)
+  uint32_t* big_hist;   // [max_rows, big_tiles_max * (RBINS + 1)] (with big)
   int32_t* big_ticket;  // [max_rows * TSTRIDE] (with big)
   int32_t big_tiles_max;
   uint64_t* ser_sum;    // [max_rows, max_chunks * SPC * NWAVE, 2] serial_kernel's segment summaries
@@ -5671,7 +5714,8 @@ int launch(xs_context* ctx, xs::Args& a, int64_t rows, int span, bool mask, bool
   a.big_ld = ctx->vocab;
   a.big_state = ctx->big_state;
   a.big_hist = ctx->big_hist;
-  a.big_hld = (int64_t)ctx->big_tiles_max * xs::RBINS;
+  a.big_hld = (int64_t)ctx->big_tiles_max * (xs::RBINS + 1);
+  a.big_tiles_max = ctx->big_tiles_max;
   a.big_ticket = ctx->big_ticket;
   a.big_tiles = (int32_t)((a.enc + xs::BTILE - 1) / xs::BTILE);
   a.big_nblk = (int32_t)(a.enc > xs::CHEAD ? (a.enc - xs::CHEAD + xs::CBLK - 1) / xs::CBLK : 0);
@@ -5748,7 +5792,7 @@ int xs_create_ex(int device, int64_t max_rows, int64_t vocab, int32_t k_max, int
     ok = ok && hipMalloc((void**)&c->big, (size_t)max_rows * 2 * vocab * sizeof(uint64_t)) == hipSuccess;
     ok = ok && hipMalloc((void**)&c->big_state, (size_t)max_rows * sizeof(xs::BigRow)) == hipSuccess;
     c->big_tiles_max = (int32_t)((vocab + xs::BTILE - 1) / xs::BTILE);
-    ok = ok && hipMalloc((void**)&c->big_hist, (size_t)max_rows * c->big_tiles_max * xs::RBINS * sizeof(uint32_t)) == hipSuccess;
+    ok = ok && hipMalloc((void**)&c->big_hist, (size_t)max_rows * c->big_tiles_max * (xs::RBINS + 1) * sizeof(uint32_t)) == hipSuccess;
     ok = ok && hipMalloc((void**)&c->big_ticket, tbytes) == hipSuccess;
     ok = ok && hipMemset(c->big_ticket, 0, tbytes) == hipSuccess;
   }
