@@ -387,6 +387,37 @@ constexpr int TSTRIDE = 32;  // one arrival ticket per 128-byte line: tickets of
 constexpr int TS_N = 1;  // whole-row path, big_ticket line: the row's sorted entries (KCUT below)
 
 struct Args {
+  // First what a workgroup reads before it has issued its loads and what its
+  // hand-off takes: the kernel arguments come through a cold scalar cache, a
+  // line at a time, and these fill its first two (one row 12.27 -> 11.88 us,
+  // a small greedy one 8.10 -> 7.77, against the same fields spread over the
+  // struct's 600 bytes).
+  int32_t n_chunks, nslots;
+  // sample_kernel's grid: rows in groups of 2^xcd_log2 (the device's XCD
+  // count, or 1), nrows of them; xcd_test 2 makes the rows of several chunks
+  // fail their placement check (a test hook)
+  int32_t xcd_log2, nrows, xcd_test;
+  // argmax_probs: every row greedy (params and uniforms unused), p_max[row] =
+  // 1 / sum exp(v - max) over the raw row
+  int32_t greedy_all;
+  int32_t n_top;
+  int32_t span;  // verify walk (0: plain batch)
+  // split launch: sample_kernel's workgroups publish and exit; finalize_kernel
+  // (one workgroup per row) finalizes every row afterwards
+  int32_t split;
+  // the serial denominator (serial_kernel), on calls with a mask or controls:
+  // bit 0, the call observes it (candidates or soft_sum), and serial_kernel
+  // finalizes its controlled rows at top_p >= 1; bit 1, the call may hold
+  // rows of top_k >= 128, and serial_kernel finalizes its controlled ones
+  int32_t serial;
+  // held_fold's re-reads are shared by the finalizing workgroup's four waves
+  // (1) or left to its first wave (0): shared when the launch's workgroups
+  // fit on the device at once, so that the waves that wait for the first
+  // wave's finalization hold no slot another workgroup needs
+  int32_t fold_shared;
+  int32_t k_max;     // the context's largest top_k (of min(top_k, enc)); larger is XS_ROW_BAD_PARAM
+  int32_t* row_ticket;  // [rows * TSTRIDE] workgroups of the row that have published (0 between calls)
+  uint64_t* rec;     // [rows, SRECW, nsp]: word i of sub-record s of a row at i * nsp + s
   const float* logits;
   int64_t ld, enc;
   const xs_row_params* params;
@@ -403,7 +434,6 @@ struct Args {
   float* soft_sum;
   float* row_max;
   double* row_lse;
-  int32_t n_top;
   int32_t* top_id;
   float* top_logprob;
   double* top_logprob64;
@@ -421,8 +451,7 @@ struct Args {
   double* probs;
   int64_t probs_ld;
   uint64_t* score_part;  // [rows, score_parts, XS_CLASS_MAX] the parts' class sums (f64 bits)
-  // verify walk (span == 0: plain batch)
-  int32_t span;
+  // verify walk
   const int32_t* drafts;
   const int32_t* budget;
   const uint8_t* done_after;  // [seqs * span] or null: committing this draft completes the grammar
@@ -432,10 +461,7 @@ struct Args {
   int32_t* committed;
   int32_t* n_committed;
   int32_t* seq_status;
-  // argmax_probs: every row greedy (params and uniforms unused), p_max[row] =
-  // 1 / sum exp(v - max) over the raw row
-  int32_t greedy_all;
-  float* p_max;
+  float* p_max;  // argmax_probs (greedy_all)
   // sparse controls (controls == nullptr: none) and what control_kernel makes
   // of them: per row a patch list of (id << 32 | final value bits) sorted by id,
   // CTL_MAX entries apart, and the first patch of every chunk (n_chunks + 1
@@ -448,11 +474,8 @@ struct Args {
   int32_t ctl_cap;      // the context's largest control list (bans plus biases of one row)
   CtlRow* ctl_row;
   int32_t* ctl_chunk;
-  // geometry + workspace
-  int32_t* row_ticket;  // [rows * TSTRIDE] workgroups of the row that have published (0 between calls)
+  // workspace
   int32_t* seq_ticket;  // [seqs * TSTRIDE] rows of the sequence that are finalized (0 between calls)
-  int32_t n_chunks, nslots;
-  int32_t k_max;     // the context's largest top_k (of min(top_k, enc)); larger is XS_ROW_BAD_PARAM
   uint64_t* big;     // [rows, 2, big_ld]: the whole-row sort's buffers (contexts with k_max > XS_K_MAX)
   int64_t big_ld;
   struct BigRow* big_state;  // [rows]: what the finalizer leaves for the whole-row kernels
@@ -464,32 +487,14 @@ struct Args {
   int32_t big_tiles_max;     // and of the context's widest row
   int32_t big_nblk;          // chain blocks per row past the first CHEAD terms
   int32_t big_cut;           // tokens only, enc <= 2^20: rows at top_k >= enc sort only p >= 2^-26
-  // the serial denominator (serial_kernel), on calls with a mask or controls:
-  // bit 0, the call observes it (candidates or soft_sum), and serial_kernel
-  // finalizes its controlled rows at top_p >= 1; bit 1, the call may hold
-  // rows of top_k >= 128, and serial_kernel finalizes its controlled ones
-  int32_t serial;
   // the finalizer's fallback to the serial sum (ser_local) for the other
   // controlled rows: rows sent there are counted (null: not counted), and
   // ser_force sends every checked row there (a test hook)
   uint32_t* ser_count;
   int32_t ser_force;
-  // split launch: sample_kernel's workgroups publish and exit; finalize_kernel
-  // (one workgroup per row) finalizes every row afterwards
-  int32_t split;
-  // sample_kernel's grid: rows in groups of 2^xcd_log2 (the device's XCD
-  // count, or 1), nrows of them; xcd_test 2 makes the rows of several chunks
-  // fail their placement check (a test hook)
-  int32_t xcd_log2, nrows, xcd_test;
-  // held_fold's re-reads are shared by the finalizing workgroup's four waves
-  // (1) or left to its first wave (0): shared when the launch's workgroups
-  // fit on the device at once, so that the waves that wait for the first
-  // wave's finalization hold no slot another workgroup needs
-  int32_t fold_shared;
   uint64_t* ser_sum;  // [rows, ser_ld, 2]: segment summaries
   uint64_t* ser_e;    // [rows, SER_NB, SEG / 2]: kept segments' terms, two f32 per word
   int64_t ser_ld;     // segments per row of ser_sum
-  uint64_t* rec;     // [rows, SRECW, nsp]: word i of sub-record s of a row at i * nsp + s
 };
 
 // The row the r-th group of n_chunks workgroups takes, for launches given a
@@ -1747,7 +1752,6 @@ XS_DEV bool fin_fast(const Args& a, const Cfg& cfg, int row, int nsub, const Ctl
   }
   // Gather the survivors into LDS, then order them by rank: a survivor's
   // position is the number of survivors above it ((key, ~id) are distinct).
-  const uint64_t floor_e = (uint64_t)tau << 32;
   int M = 0;
   auto put = [&](uint64_t e, bool ok) __attribute__((always_inline)) {
     const uint64_t b = __ballot(ok);
@@ -1764,7 +1768,7 @@ XS_DEV bool fin_fast(const Args& a, const Cfg& cfg, int row, int nsub, const Ctl
     int c = 0;
 #pragma unroll
     for (int j = 0; j < EPRE; j++) {
-      ok[j] = j < cnt && E[j] >= floor_e;
+      ok[j] = j < cnt && pk_key(E[j]) >= tau;
       c += ok[j] ? 1 : 0;
     }
     const int incl = wave_incl_scan(c);
@@ -1783,7 +1787,7 @@ XS_DEV bool fin_fast(const Args& a, const Cfg& cfg, int row, int nsub, const Ctl
   // Many of them in one sub-record, or more survivors than the list holds:
   // the general path's gather_survivors.
   const bool srt = (hf & 4u) != 0;
-  int lim = (srt && E[EPRE - 1] < floor_e) ? EPRE : cnt;
+  int lim = (srt && pk_key(E[EPRE - 1]) < tau) ? EPRE : cnt;
   if (XS_RARE(M > SURV || __ballot(lim > 2 * EPRE))) return false;
 #pragma unroll 1
   for (int j0 = EPRE; __ballot(j0 < lim); j0 += 4) {
@@ -1792,8 +1796,8 @@ XS_DEV bool fin_fast(const Args& a, const Cfg& cfg, int row, int nsub, const Ctl
     for (int u = 0; u < 4; u++)  // (clamped inside the sub-record, not guarded: all four in flight)
       e[u] = ld_sub<LOC>(rowrec + (int64_t)(SHDR + min(j0 + u, CAPW - 1)) * nsp + lane);
 #pragma unroll
-    for (int u = 0; u < 4; u++) put(e[u], j0 + u < lim && e[u] >= floor_e);
-    if (srt && j0 + 3 < lim && e[3] < floor_e) lim = j0;
+    for (int u = 0; u < 4; u++) put(e[u], j0 + u < lim && pk_key(e[u]) >= tau);
+    if (srt && j0 + 3 < lim && pk_key(e[3]) < tau) lim = j0;
   }
   if (XS_RARE(M > SURV)) return false;
   F.expt[lane] = et;
