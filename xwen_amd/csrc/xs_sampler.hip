@@ -4204,6 +4204,14 @@ __global__ __launch_bounds__(BLOCK) void score_kernel(Args a, int np) {
 // pass a power of two or a flag is set).  The row's last workgroup (the
 // arrival ticket, as in sample_kernel) walks the summaries and finalizes the
 // row with the serial sum as its denominator.
+// A workgroup of SER_G groups of BLOCK lanes, each group SER_SPG of its chunk's
+// slots: bound by the terms' arithmetic and its latencies, and at two
+// four-wave workgroups a CU (their LDS allows no more) the SIMDs were half
+// idle (32 masked rows with weights: serial_kernel 77 -> 68 us with two
+// groups; with four, a workgroup fills a CU's registers alone and the launch
+// takes two rounds: 101 us).
+constexpr int SER_G = 2;
+constexpr int SER_SPG = SPC / SER_G;
 struct SerLds {
   double expt[64];
   double segsum[SPC * NWAVE];  // exact sums of the chunk's segments, row order (short exp)
@@ -4212,8 +4220,8 @@ struct SerLds {
   uint32_t R[SPC * NWAVE][2];  // units at the segment's lower binade and the next
   uint32_t meta[SPC * NWAVE];  // summary word 1's high half, without the kept slot
   uint64_t kmask;              // segments of the chunk that keep their terms
-  float qd[NWAVE][SER_QCAP];   // per wave: exp arguments queued for the correctly rounded exp
-  uint8_t qt[NWAVE][SER_QCAP]; // and their segments
+  float qd[SER_G * NWAVE][SER_QCAP];   // per wave: exp arguments queued for the correctly rounded exp
+  uint8_t qt[SER_G * NWAVE][SER_QCAP]; // and their segments
   float m_s;
   int32_t ok, last, nb, kbase;
 };
@@ -4239,10 +4247,12 @@ __device__ __attribute__((noinline)) float4 cr_exp4(float4 d, const double* T) {
 }
 
 template <bool HAS_MASK, bool HAS_CTL>
-__global__ __launch_bounds__(BLOCK) void serial_kernel(Args a) {
+__global__ __launch_bounds__(SER_G * BLOCK) void serial_kernel(Args a) {
   __shared__ SerLds Ls;
   __shared__ SerTail St;
-  const int tid = threadIdx.x, lane = lane_id(), wave = wave_id();
+  const int tid = threadIdx.x, lane = lane_id(), wv = wave_id();
+  const int pos = tid & (BLOCK - 1), wave = wv & (NWAVE - 1);  // the thread's float4 of a slot, and the slot's quarter
+  const int j0 = (wv / NWAVE) * SER_SPG;                        // its group's first slot of the chunk
   const int nc = a.n_chunks;
   const int row = blockIdx.x / nc;
   const int chunk = blockIdx.x - row * nc;
@@ -4261,7 +4271,7 @@ __global__ __launch_bounds__(BLOCK) void serial_kernel(Args a) {
   // the row max (sample_kernel's headers) and the exact sum before this
   // chunk: their loads go out first, the chunk's after them
   uint64_t h0[GMAX], h1[GMAX], h3[GMAX];
-  if (wave == 0) {
+  if (wv == 0) {
 #pragma unroll
     for (int gi = 0; gi < GMAX; gi++) {
       const int sub = gi * 64 + lane;
@@ -4275,18 +4285,18 @@ __global__ __launch_bounds__(BLOCK) void serial_kernel(Args a) {
       h1[gi] = before ? h1[gi] : 0ull;
     }
   }
-  v4f q[SPC];
-  uint32_t mw[SPC];
+  v4f q[SER_SPG];
+  uint32_t mw[SER_SPG];
 #pragma unroll
-  for (int j = 0; j < SPC; j++) {
-    const int f = min((s0 + j) * BLOCK + tid, fmax);
-    q[j] = rp4[f];
-    if (HAS_MASK) mw[j] = mrow[f >> 3];
+  for (int i = 0; i < SER_SPG; i++) {
+    const int f = min((s0 + j0 + i) * BLOCK + pos, fmax);
+    q[i] = rp4[f];
+    if (HAS_MASK) mw[i] = mrow[f >> 3];
   }
   CtlRow cr{};
   if (HAS_CTL) cr = a.ctl_row[row];
   if (tid < 64) Ls.expt[tid] = (&kExpT[0][0])[tid];
-  if (wave == 0) {
+  if (wv == 0) {
     float mv = -INFINITY;
     uint32_t fw = 0;
 #pragma unroll
@@ -4329,28 +4339,29 @@ __global__ __launch_bounds__(BLOCK) void serial_kernel(Args a) {
       pl = a.patch + (int64_t)row * a.ctl_cap;
     }
 #pragma unroll
-    for (int j = 0; j < SPC; j++) {
-      float x[4] = {q[j].x, q[j].y, q[j].z, q[j].w};
+    for (int i = 0; i < SER_SPG; i++) {
+      const int j = j0 + i;
+      float x[4] = {q[i].x, q[i].y, q[i].z, q[i].w};
       if (HAS_MASK) {
-        const uint32_t bits = mw[j] >> ((((s0 + j) * BLOCK + tid) & 7) * 4);
+        const uint32_t bits = mw[i] >> ((((s0 + j) * BLOCK + pos) & 7) * 4);
 #pragma unroll
         for (int e = 0; e < 4; e++)
           if (!((bits >> e) & 1u)) x[e] = -INFINITY;
       }
       if (j >= ns || (s0 + j + 1) * SLOT > enc) {
-        const int id0 = (s0 + j) * SLOT + 4 * tid;
+        const int id0 = (s0 + j) * SLOT + 4 * pos;
 #pragma unroll
         for (int e = 0; e < 4; e++)
           if (j >= ns || id0 + e >= enc) x[e] = -INFINITY;
       }
-      if (ctl_on) ctl_slot(x, (s0 + j) * SLOT, tid, pl, pc, phi, cr.pull_id, cr.pull_val, cr.force_id, cr.force_val);
+      if (ctl_on) ctl_slot(x, (s0 + j) * SLOT, pos, pl, pc, phi, cr.pull_id, cr.pull_val, cr.force_id, cr.force_val);
       float dv[4], t = 0.0f;
 #pragma unroll
       for (int e = 0; e < 4; e++) {
         dv[e] = (cfg.scale ? x[e] * cfg.inv : x[e]) - m_s;
         t += fast_expf(dv[e]);
       }
-      q[j] = v4f{dv[0], dv[1], dv[2], dv[3]};
+      q[i] = v4f{dv[0], dv[1], dv[2], dv[3]};
       const double ssum = wave_sumd((double)t);
       const bool any = __ballot(dv[0] >= -104.0f || dv[1] >= -104.0f || dv[2] >= -104.0f || dv[3] >= -104.0f) != 0;
       if (lane == 0) {
@@ -4360,7 +4371,7 @@ __global__ __launch_bounds__(BLOCK) void serial_kernel(Args a) {
     }
   }
   __syncthreads();
-  if (ok && wave == 0) {  // exact prefixes, in row order
+  if (ok && wv == 0) {  // exact prefixes, in row order
     const double v = Ls.segsum[lane];
     double inc = v;
 #pragma unroll
@@ -4380,22 +4391,23 @@ __global__ __launch_bounds__(BLOCK) void serial_kernel(Args a) {
     // terms too: d in [-104, -87)); the settled units stay in registers until
     // the queue is empty
     int qn = 0;
-    uint32_t fr0[SPC], fr1[SPC];
-    if (lane < SPC) {
-      const int t = lane * NWAVE + wave;
+    uint32_t fr0[SER_SPG], fr1[SER_SPG];
+    if (lane < SER_SPG) {
+      const int t = (j0 + lane) * NWAVE + wave;
       Ls.R[t][0] = 0u;
       Ls.R[t][1] = 0u;
     }
 #pragma unroll
-    for (int j = 0; j < SPC; j++) {
-      fr0[j] = fr1[j] = 0u;
+    for (int i = 0; i < SER_SPG; i++) {
+      const int j = j0 + i;
+      fr0[i] = fr1[i] = 0u;
       if (j < ns) {
         const int t = j * NWAVE + wave;
         const double X0 = Ls.segpre[t];
         const int FB = f32_field((float)(X0 * (1.0 - SER_DELTA)));
         const bool two = f32_field((float)(X0 * (1.0 + SER_DELTA))) != FB;
         if (lane == 0) Ls.meta[t] |= (uint32_t)FB | (two ? SM_TWO : 0u);
-        const float dv[4] = {q[j].x, q[j].y, q[j].z, q[j].w};
+        const float dv[4] = {q[i].x, q[i].y, q[i].z, q[i].w};
         uint32_t r0 = 0, r1 = 0;
 #pragma unroll
         for (int k = 0; k < 4; k++) {
@@ -4411,32 +4423,32 @@ __global__ __launch_bounds__(BLOCK) void serial_kernel(Args a) {
           const uint64_t b = __ballot(amb);
           if (b) {
             if (qn + 64 > SER_QCAP) {
-              ser_flush(Ls, wave, qn, Ls.expt);
+              ser_flush(Ls, wv, qn, Ls.expt);
               qn = 0;
             }
-            const int pos = qn + lanes_below(b);
+            const int at = qn + lanes_below(b);
             if (amb) {
-              Ls.qd[wave][pos] = dv[k];
-              Ls.qt[wave][pos] = (uint8_t)t;
+              Ls.qd[wv][at] = dv[k];
+              Ls.qt[wv][at] = (uint8_t)t;
             }
             qn += __popcll(b);
           }
         }
-        fr0[j] = wave_sum_u32(r0);
-        fr1[j] = wave_sum_u32(r1);
+        fr0[i] = wave_sum_u32(r0);
+        fr1[i] = wave_sum_u32(r1);
       }
     }
-    ser_flush(Ls, wave, qn, Ls.expt);
+    ser_flush(Ls, wv, qn, Ls.expt);
     if (lane == 0) {
 #pragma unroll
-      for (int j = 0; j < SPC; j++) {
-        Ls.R[j * NWAVE + wave][0] += fr0[j];
-        Ls.R[j * NWAVE + wave][1] += fr1[j];
+      for (int i = 0; i < SER_SPG; i++) {
+        Ls.R[(j0 + i) * NWAVE + wave][0] += fr0[i];
+        Ls.R[(j0 + i) * NWAVE + wave][1] += fr1[i];
       }
     }
   }
   __syncthreads();
-  if (ok && wave == 0) {
+  if (ok && wv == 0) {
     // segments that keep their terms: nonzero ones where the exact sum may
     // pass a power of two, or with a half-way term (lane t: segment t); one
     // reservation of side-buffer slots for the workgroup
@@ -4462,12 +4474,13 @@ __global__ __launch_bounds__(BLOCK) void serial_kernel(Args a) {
     const uint64_t km = Ls.kmask;
     const int kbase = Ls.kbase;
 #pragma unroll
-    for (int j = 0; j < SPC; j++) {
+    for (int i = 0; i < SER_SPG; i++) {
+      const int j = j0 + i;
       const int t = j * NWAVE + wave;
       const int idx = kbase + __popcll(km & ((1ull << t) - 1ull));
       uint32_t ones = 0u;  // the segment's single half-way terms (SM_ONE0, ...)
       if (j < ns && ((km >> t) & 1ull) && idx < SER_NB) {  // a kept segment: its terms correctly rounded
-        const float4 e = cr_exp4(make_float4(q[j].x, q[j].y, q[j].z, q[j].w), Ls.expt);
+        const float4 e = cr_exp4(make_float4(q[i].x, q[i].y, q[i].z, q[i].w), Ls.expt);
         uint64_t* const dst = skeep + (int64_t)idx * (SEG / 2) + 2 * lane;
         st_agent(dst, (uint64_t)__float_as_uint(e.x) | ((uint64_t)__float_as_uint(e.y) << 32));
         st_agent(dst + 1, (uint64_t)__float_as_uint(e.z) | ((uint64_t)__float_as_uint(e.w) << 32));
@@ -4505,22 +4518,22 @@ __global__ __launch_bounds__(BLOCK) void serial_kernel(Args a) {
   if (ok) {
     const int nseg = a.nslots * NWAVE;
     const int nbl = min(min(Ls.nb, SER_NB), SER_LDS);
-    for (int i = tid; i < nbl * (SEG / 2); i += BLOCK)
+    for (int i = tid; i < nbl * (SEG / 2); i += SER_G * BLOCK)
       reinterpret_cast<uint64_t*>(&St.w.ev[0][0])[i] = ld_agent(&skeep[i]);
     uint32_t sb = 0;  // the running sum's bits, from +0
 #pragma unroll 1
     for (int w0 = 0; w0 < nseg; w0 += SER_WIN) {
       const int wn = min(SER_WIN, nseg - w0);
-      for (int i = tid; i < 2 * wn; i += BLOCK) (&St.w.sum[0][0])[i] = ld_agent(&ssum[2 * (int64_t)w0 + i]);
+      for (int i = tid; i < 2 * wn; i += SER_G * BLOCK) (&St.w.sum[0][0])[i] = ld_agent(&ssum[2 * (int64_t)w0 + i]);
       __syncthreads();
-      if (wave == 0)
+      if (wv == 0)
         sb = ser_walk<HAS_MASK, HAS_CTL>(a, cfg, row, sb, St.w.sum, w0, wn, St.w.ev, nbl, skeep, m_s, Ls.expt,
                                          St.w.ev[SER_LDS]);
       __syncthreads();
     }
     S_ser = __uint_as_float(sb);
   }
-  if (wave != 0) return;
+  if (wv != 0) return;
   finalize_row<HAS_MASK, false, HAS_CTL, true>(a, cfg, row, rowrec, nsp, nsub, rowp, mrow, St.tl.fin, S_ser);
   if (a.span > 0 && !deferred(cfg, St.tl.fin)) verify_walk(a, row);
 }
@@ -5738,7 +5751,7 @@ void launch2(xs_context* ctx, xs::Args& a, int64_t rows, dim3 g1, dim3 gs, const
                        xs::RowOrder<false>{});
   }
   if (a.split) hipLaunchKernelGGL((xs::finalize_kernel<M, S, C>), dim3((unsigned)rows), dim3(xs::BLOCK), 0, ctx->stream, a);
-  if ((M || C) && a.serial) hipLaunchKernelGGL((xs::serial_kernel<M, C>), g1, dim3(xs::BLOCK), 0, ctx->stream, a);
+  if ((M || C) && a.serial) hipLaunchKernelGGL((xs::serial_kernel<M, C>), g1, dim3(xs::SER_G * xs::BLOCK), 0, ctx->stream, a);
   // a call that may hold top_k >= 128 on a context sized for it: the
   // whole-row kernels (rows not drawn there return at once)
   if (a.big && !a.greedy_all && a.k_max > XS_K_MAX) {
