@@ -54,3 +54,20 @@ def test_calls_share_the_buffers(oracle):
         assert s.sample_controlled(xd, ctl, u).tolist() == _want(oracle, x, opts, u, ctl)
     assert s.sample(torch.as_tensor(x).cuda(), u).tolist() == _want(oracle, x, opts, u)
     assert err.value.status.tolist() == [0, 1, 0]
+
+
+def test_greedy_takes_fewer_uniforms(oracle):
+    """Greedy rows ignore their uniforms, so a short array is as good as a full
+    one; a stochastic sampler refuses it, and both refuse an empty one."""
+    from xwen_amd import sampler as xsm
+    x = np.random.default_rng(6).standard_normal((4, V)).astype(np.float32)
+    xd = torch.as_tensor(x).cuda()
+    for opts in (xsm.SamplerOptions(temperature=0.0), xsm.SamplerOptions(temperature=0.7, top_k=1)):
+        s = xsm.Sampler(opts, [0], V, max_rows=4)
+        for u in ([0.5], np.zeros(3, np.float32), np.zeros(9, np.float32)):
+            assert s.sample(xd, u).tolist() == x.argmax(1).tolist()
+        with pytest.raises(ValueError):
+            s.sample(xd, [])
+    s = xsm.Sampler(xsm.SamplerOptions(temperature=0.7), [0], V, max_rows=4)
+    with pytest.raises(ValueError):
+        s.sample(xd, [0.5])

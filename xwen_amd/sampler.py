@@ -560,10 +560,12 @@ class Sampler:
         b = self._bufs
         if rows > b["rows"]:
             b = self._bufs = self._buffers(rows)
-        u = np.asarray(uniforms, np.float32).reshape(-1)
+        u = np.asarray(uniforms, np.float32).reshape(-1)[:rows]
         if u.size < rows:
-            raise ValueError(f"{rows} rows need as many uniforms, got {u.size}")
-        b["u"][:rows] = u[:rows]
+            if u.size == 0 or not self.opts.is_greedy():  # (greedy rows ignore theirs)
+                raise ValueError(f"{rows} rows need as many uniforms, got {u.size}")
+            u = np.concatenate([u, np.zeros(rows - u.size, np.float32)])
+        b["u"][:rows] = u
         p = self._row_params(rows, logits.device)
         allowed = None if ctl is None else ctl.allowed
         controls = None
