@@ -71,3 +71,49 @@ def test_greedy_takes_fewer_uniforms(oracle):
     s = xsm.Sampler(xsm.SamplerOptions(temperature=0.7), [0], V, max_rows=4)
     with pytest.raises(ValueError):
         s.sample(xd, [0.5])
+
+
+def test_a_call_left_in_an_exception_keeps_its_block(oracle, monkeypatch):
+    """A call interrupted after its launch leaves kernels that still read its
+    uniforms and write its tokens: the next call, on another stream and before
+    them, must not share their block, and the block is given back once they
+    have run."""
+    from xwen_amd import sampler as xsm
+    rng = np.random.default_rng(7)
+    opts = xsm.SamplerOptions(temperature=0.9, top_k=20, top_p=0.95)
+    s = xsm.Sampler(opts, [0], V, max_rows=4)
+    x = rng.standard_normal((4, V)).astype(np.float32) * np.float32(2.0)
+    xd = torch.as_tensor(x).cuda()
+    u1, u2 = workloads.uniforms(rng, 4), workloads.uniforms(rng, 4)
+    want1, want2 = _want(oracle, x, opts, u1), _want(oracle, x, opts, u2)
+    assert s.sample(xd, u2).tolist() == want2  # (options packed, buffers taken once)
+    torch.cuda.synchronize()
+    launch = xsm.sample_batch
+    first = {}
+
+    def interrupted(*a, out, **kw):
+        torch.cuda._sleep(50_000_000)  # the launch waits on its stream: 20 ms or more
+        launch(*a, out=out, **kw)
+        first.update(u=a[3], token=out.token)
+        raise KeyboardInterrupt
+
+    slow = torch.cuda.Stream()
+    with torch.cuda.stream(slow):
+        monkeypatch.setattr(xsm, "sample_batch", interrupted)
+        with pytest.raises(KeyboardInterrupt):
+            s.sample(xd, u1)
+        monkeypatch.setattr(xsm, "sample_batch", launch)
+        assert len(s._stuck) == 1 and s._bufs is None
+    fast = torch.cuda.Stream()
+    with torch.cuda.stream(fast):
+        got = s.sample(xd, u2)
+    assert got.tolist() == want2
+    assert s._bufs["host"].data_ptr() != first["u"].data_ptr()
+    assert first["u"].numpy().view(np.float32)[:4].tolist() == u1.tolist()  # still what that launch will read
+    slow.synchronize()
+    assert first["token"].numpy()[:4].tolist() == want1
+    assert s.sample(xd, u2).tolist() == want2 and not s._stuck
+    with pytest.raises(xsm._lib.XsError):  # a refused call (more rows than the context holds)
+        s.sample(torch.zeros((5, V), device="cuda"), np.zeros(5, np.float32))
+    for u, want in ((u1, want1), (u2, want2)):
+        assert s.sample(xd, u).tolist() == want and not s._stuck

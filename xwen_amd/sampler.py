@@ -501,6 +501,7 @@ class Sampler:
         self.ctx = Context(max_rows, encodable, k_max=max(k_max, _lib.K_MAX), device=device)
         self.device = f"cuda:{device}"
         self._bufs = self._buffers(max_rows)
+        self._stuck = []  # (stream, block, params) of calls that ended in an exception
         self._params = None
 
     @staticmethod
@@ -509,12 +510,28 @@ class Sampler:
         uniforms it draws from and the tokens and statuses it leaves, in pinned
         memory that the kernels read and write in place, so that a call makes
         no copies (4 rows: 89 us a call with three uploads, two allocations and
-        two read-backs, 34 without).  A call ends with its stream's
-        synchronize, so the next one may reuse them."""
+        two read-backs, 34 without).  A call that ends with its stream's
+        synchronize leaves its block to the next one (_take_buffers)."""
         torch = _torch()
         host = torch.empty((3, rows), dtype=torch.int32, pin_memory=True)
         view = host.numpy()
         return {"rows": rows, "host": host, "u": view[0].view(np.float32), "token": view[1], "status": view[2]}
+
+    def _take_buffers(self, rows):
+        """A block that no launch reads or writes.  One that a call left in an
+        exception (after its launch, or in its wait) may still be in use: it is
+        kept until its stream has run dry, and never taken again before."""
+        self._free_stuck(None)
+        b, self._bufs = self._bufs, None
+        if b is None or b["rows"] < rows:
+            b = self._buffers(max(rows, self.ctx.max_rows))
+        return b
+
+    def _free_stuck(self, drained):
+        """Give back the blocks of interrupted calls whose stream has run dry
+        (`drained`: one known to have)."""
+        if self._stuck:
+            self._stuck = [e for e in self._stuck if e[0] != drained and not e[0].query()]
 
     def _row_params(self, rows, device):
         """xs_row_params for every row of a call, kept on the device while the
@@ -557,15 +574,11 @@ class Sampler:
             logits = padded
         if uniforms is None:
             uniforms = self.next_uniforms(rows)
-        b = self._bufs
-        if rows > b["rows"]:
-            b = self._bufs = self._buffers(rows)
         u = np.asarray(uniforms, np.float32).reshape(-1)[:rows]
         if u.size < rows:
             if u.size == 0 or not self.opts.is_greedy():  # (greedy rows ignore theirs)
                 raise ValueError(f"{rows} rows need as many uniforms, got {u.size}")
             u = np.concatenate([u, np.zeros(rows - u.size, np.float32)])
-        b["u"][:rows] = u
         p = self._row_params(rows, logits.device)
         allowed = None if ctl is None else ctl.allowed
         controls = None
@@ -573,14 +586,22 @@ class Sampler:
             controls = controls_tensor([ctl] * rows, logits.device)
         stream = torch.cuda.current_stream(self.ctx.device)
         self.ctx.bind_current_stream()
+        b = self._take_buffers(rows)
+        b["u"][:rows] = u
         host = b["host"]
-        sample_batch(self.ctx, logits, p, host[0], enc=self.encodable_, width=width, allowed=allowed,
-                     controls=controls, out=Draws(token=host[1], status=host[2]))
-        stream.synchronize()
-        st = b["status"][:rows]
+        try:
+            sample_batch(self.ctx, logits, p, host[0], enc=self.encodable_, width=width, allowed=allowed,
+                         controls=controls, out=Draws(token=host[1], status=host[2]))
+            stream.synchronize()
+        except BaseException:
+            self._stuck.append((stream, b, p))
+            raise
+        token, st = b["token"][:rows].astype(np.int64), b["status"][:rows].copy()
+        self._bufs = b
+        self._free_stuck(stream)
         if st.any():
-            raise SampleError(st.copy())
-        return b["token"][:rows].astype(np.int64)
+            raise SampleError(st)
+        return token
 
     def sample(self, logits, uniforms=None):
         return self.sample_controlled(logits, None, uniforms)
