@@ -269,3 +269,35 @@ def test_tokens_only_rows_sort_what_the_sums_see(bigctx, oracle):
             assert (full["status"] == 0).all() and (toks["status"] == 0).all()
             np.testing.assert_array_equal(toks["token"], full["token"])
             check_rows(oracle, x, T, K, Pm, U, full, mask=m, label="tokens only vs full sort")
+
+
+@pytest.mark.parametrize("v", [3_001, 4_096, 40_003])
+@pytest.mark.parametrize("shape", ["masked", "sharp", "flat", "half", "runs"])
+def test_rows_of_equal_digits(oracle, v, shape):
+    """Counting passes whose waves hold one digit in most lanes (a mask's or a low
+    temperature's +0, a flat row), in half of them, and in some waves only; the
+    last step of a tile partly filled; with candidates and tokens only."""
+    from xwen_amd import sampler as xsm
+    rng = np.random.default_rng(v)
+    rows, k = 6, 300
+    ld = (v + 3) // 4 * 4
+    x = rng.normal(0, 0.01 if shape == "flat" else 3, (rows, ld)).astype(np.float32)
+    T, mask = 0.1 if shape == "sharp" else 0.9, None
+    if shape == "half":  # every other id left out
+        x[:, :v:2] = -np.inf
+    elif shape == "runs":  # whole waves left out, the one beside them not
+        x[:, (np.arange(ld) // 256) % 2 == 1] = -np.inf
+    elif shape == "masked":
+        allow = rng.random((rows, v)) < 0.15
+        mask = workloads.pack_mask(allow)
+    U = workloads.uniforms(rng, rows)
+    P = np.array([0.9, 1.0, 0.95] * 2)
+    ctx = xsm.Context(max_rows=rows, vocab=v, k_max=v)
+    ctx.bind_current_stream()
+    for K in (np.full(rows, k), np.full(rows, v)):
+        d = run_sample(ctx, x, T, K, P, U, enc=v, mask=mask, cand_k=v)
+        assert (d["status"] == 0).all(), d["status"]
+        check_rows(oracle, x, np.full(rows, T), K, P, U, d, enc=v, mask=mask, margins=False, label=f"{v} {shape}")
+        t = run_sample(ctx, x, T, K, P, U, enc=v, mask=mask, cand_k=0, stats=False)
+        assert t["token"].tolist() == d["token"].tolist() and (t["status"] == 0).all()
+    ctx.close()

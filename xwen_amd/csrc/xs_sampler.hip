@@ -4968,11 +4968,33 @@ XS_DEV uint64_t digit_peers(uint32_t d, bool valid) {
   return m;
 }
 XS_DEV uint64_t lanes_below() { return (1ull << lane_id()) - 1ull; }
-// Count this lane's digit.  (One LDS add a lane: grouping equal digits first
-// by digit_peers costs some 50 instructions to save the conflicts, which 256
-// digits seldom make, and bound the counting passes: 64 rows of 248,320 ids,
-// big_hist_kernel 24 -> 17 us, big_scatter_kernel 37 -> 33.)
-XS_DEV void count_digit(uint32_t* cnt, uint32_t d, bool valid) {
+// Count this lane's digit: one LDS add a lane.  Grouping equal digits first
+// (digit_peers) costs some 50 instructions a step and bounded the counting
+// passes of ordinary rows, whose 256 digits seldom conflict (64 rows of
+// 248,320 ids cut at 2^-26: big_hist_kernel 24 -> 17 us without it,
+// big_scatter_kernel 37 -> 33).  Rows with many equal keys are not ordinary:
+// the +0 of the ids a mask leaves out, of a low temperature's tail, a flat
+// row's leading digits.  There a wave whose first step holds one digit in half
+// its lanes or more (digits_alike) adds that digit's lanes at once (16 rows of
+// 248,320 ids at top_k 1,000 with their candidates: masked 369 -> 315 us, at
+// T 0.1 276 -> 222, flat 247 -> 230; plain rows stay at 290, and 302 with the
+// grouping in every wave).  A cut row's keys hold no +0, and its waves are not
+// asked (64 top-p-only rows: 320 us, 324 asked).
+XS_DEV bool digits_alike(uint32_t d, bool valid) {
+  const uint64_t v = __ballot(valid);
+  if (v == 0ull) return false;
+  return __popcll(__ballot(valid && d == rdl(d, (int)__builtin_ctzll(v)))) >= 32;
+}
+XS_DEV void count_digit(uint32_t* cnt, uint32_t d, bool valid, bool alike) {
+  if (alike) {
+    const uint64_t v = __ballot(valid);
+    if (v == 0ull) return;
+    const int l = (int)__builtin_ctzll(v);
+    const bool same = valid && d == rdl(d, l);
+    const uint64_t b = __ballot(same);
+    if (lane_id() == l) atomicAdd(&cnt[d], (uint32_t)__popcll(b));
+    valid = valid && !same;
+  }
   if (valid) atomicAdd(&cnt[d], 1u);
 }
 
@@ -5082,6 +5104,7 @@ __global__ __launch_bounds__(BLOCK) void big_key_kernel(Args a) {
   __syncthreads();
   uint64_t* const A = a.big + (int64_t)row * 2 * a.big_ld;
   const int lane = lane_id(), wave = wave_id();
+  bool alike = false;
   uint32_t needs = 0u;  // a cut row: bit 4j + e, element e of slot j is left for the exact p
   const float invS = 1.0f / S;
   if (cut && tid < SPT * NWAVE) seg[tid] = 0;  // (absent slots)
@@ -5116,10 +5139,10 @@ __global__ __launch_bounds__(BLOCK) void big_key_kernel(Args a) {
     }
     uint32_t k[4];
 #pragma unroll
-    for (int e = 0; e < 4; e++) {
-      k[e] = pkey(exact_p(x[e], cfg, m_s, S, expt));
-      count_digit(hist, rdigit(k[e], 0), id0 + e < enc);
-    }
+    for (int e = 0; e < 4; e++) k[e] = pkey(exact_p(x[e], cfg, m_s, S, expt));
+    if (j == 0) alike = digits_alike(rdigit(k[0], 0), id0 < enc);
+#pragma unroll
+    for (int e = 0; e < 4; e++) count_digit(hist, rdigit(k[e], 0), id0 + e < enc, alike);
     if (id0 + 3 < enc) {
 #pragma unroll
       for (int e = 0; e < 4; e++) A[id0 + e] = ((uint64_t)k[e] << 32) | (uint32_t)(id0 + e);
@@ -5167,7 +5190,7 @@ __global__ __launch_bounds__(BLOCK) void big_key_kernel(Args a) {
       const uint2 it = ent[v ? i : 0];
       uint32_t k = pkey(exact_p(__uint_as_float(it.x), cfg, m_s, S, expt));
       if (k > KCUT) k = KSENT;  // (below the cut after all)
-      count_digit(hist, rdigit(k, 0), v && k != KSENT);
+      count_digit(hist, rdigit(k, 0), v && k != KSENT, false);  // (a cut row has no +0)
       if (v) A[tile * BTILE + i] = ((uint64_t)k << 32) | it.y;
     }
   }
@@ -5193,7 +5216,9 @@ __global__ __launch_bounds__(BLOCK) void big_hist_kernel(Args a, int pass) {
   __shared__ int32_t last;
   const int row = blockIdx.x / a.big_tiles, tile = blockIdx.x % a.big_tiles;
   Cfg cfg;
-  if (!big_live(a, row, cfg)) return;
+  const BigRow* br = big_live(a, row, cfg);
+  if (!br) return;
+  const bool cut = a.big_cut && br->kk == (int)a.enc;
   const int ntl = big_sorted_tiles(a, row);  // the tiles the first pass filled
   if (tile >= ntl) return;
   const int tid = threadIdx.x;
@@ -5208,9 +5233,15 @@ __global__ __launch_bounds__(BLOCK) void big_hist_kernel(Args a, int pass) {
     k[s] = i < nt ? src[2 * i + 1] : 0u;
   }
   hist[tid] = 0u;
+  const bool alike = !cut && digits_alike(rdigit(k[0], pass), tid < nt);
   __syncthreads();
+  if (alike) {
 #pragma unroll
-  for (int s = 0; s < EPL; s++) count_digit(hist, rdigit(k[s], pass), s * BLOCK + tid < nt);
+    for (int s = 0; s < EPL; s++) count_digit(hist, rdigit(k[s], pass), s * BLOCK + tid < nt, true);
+  } else {
+#pragma unroll
+    for (int s = 0; s < EPL; s++) count_digit(hist, rdigit(k[s], pass), s * BLOCK + tid < nt, false);
+  }
   __syncthreads();
   big_counts(a, row, tile, hist[tid], s4, last, ntl);
 }
@@ -5224,7 +5255,9 @@ __global__ __launch_bounds__(BLOCK) void big_scatter_kernel(Args a, int pass) {
   __shared__ uint64_t ent[NWAVE][QW];     // per wave: its quarter of the tile
   const int row = blockIdx.x / a.big_tiles, tile = blockIdx.x % a.big_tiles;
   Cfg cfg;
-  if (!big_live(a, row, cfg)) return;
+  const BigRow* br = big_live(a, row, cfg);
+  if (!br) return;
+  const bool cut = a.big_cut && br->kk == (int)a.enc;
   // the first pass reads what the key kernel left of the tile's ids (in id
   // order, KSENT on a few left out), the others the entries it sorted; each
   // wave takes a quarter of them
@@ -5251,10 +5284,13 @@ __global__ __launch_bounds__(BLOCK) void big_scatter_kernel(Args a, int pass) {
 #pragma unroll
   for (int i = lane; i < RBINS; i += 64) cnt[wave][i] = 0u;
   wave_lds_sync();
+  bool alike = false;
 #pragma unroll 1
   for (int s = 0; s < steps; s++) {
     const uint32_t key = (uint32_t)(ent[wave][s * 64 + lane] >> 32);
-    count_digit(cnt[wave], rdigit(key, pass), q0 + s * 64 + lane < nt && key != KSENT);
+    const bool valid = q0 + s * 64 + lane < nt && key != KSENT;
+    if (s == 0 && !cut) alike = digits_alike(rdigit(key, pass), valid);
+    count_digit(cnt[wave], rdigit(key, pass), valid, alike);
   }
   __syncthreads();
   // each wave's first position of every digit (thread t: digit t)
