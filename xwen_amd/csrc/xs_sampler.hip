@@ -6048,6 +6048,8 @@ int sample_impl(xs_context* ctx, const xs_sample_args* in, bool clear_tickets) {
   a.n_chunks = chunks_for(in->enc);
   a.nslots = (int32_t)slots_for(in->enc);
   a.rec = ctx->rec;
+  const int np = (a.probs || a.n_class > 0) ? xs::score_parts(a.nslots) : 1;  // score_kernel's workgroups a row
+  if (scores && in->rows * (int64_t)np > 0x7FFFFFFF) return XS_ERR_CAPACITY;
   if (clear_tickets && in->rows > 0) {
     const int64_t n = in->rows * xs::TSTRIDE;
     hipLaunchKernelGGL(xs::zero_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, ctx->stream,
@@ -6103,8 +6105,6 @@ int sample_impl(xs_context* ctx, const xs_sample_args* in, bool clear_tickets) {
   // fails the caller's row)
   a.token = in->token;
   a.status = in->status;
-  const int np = (a.probs || a.n_class > 0) ? xs::score_parts(a.nslots) : 1;
-  if (in->rows * (int64_t)np > 0x7FFFFFFF) return XS_ERR_CAPACITY;
   hipLaunchKernelGGL(xs::score_kernel, dim3((unsigned)(in->rows * np)), dim3(xs::BLOCK), 0, ctx->stream, a, np);
   return hipGetLastError() == hipSuccess ? XS_OK : XS_ERR_HIP;
 }
