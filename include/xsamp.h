@@ -103,7 +103,7 @@ typedef struct {
  * rows of up to `vocab` encodable ids (<= 1,048,576) and min(top_k, enc) <=
  * k_max (any k_max >= 0; the reference's top_k is an unbounded usize, and
  * INT32_MAX serves every top_k).  k_max above XS_K_MAX adds the whole-row
- * path's buffers, 16 bytes per row and id plus 1 KiB per row and 4,096 ids
+ * path's buffers, 16 bytes per row and id plus 1,028 per row and 4,096 ids
  * (33 MB for 8 rows of 248,320), and every sampling call on such a context
  * then launches the whole-row kernels too (rows that do not take that path
  * return at once: about 33 us more per call when no row does), unless the

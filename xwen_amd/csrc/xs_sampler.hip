@@ -389,9 +389,10 @@ constexpr int TS_N = 1;  // whole-row path, big_ticket line: the row's sorted en
 struct Args {
   // First what a workgroup reads before it has issued its loads and what its
   // hand-off takes: the kernel arguments come through a cold scalar cache, a
-  // line at a time, and these fill its first two (one row 12.27 -> 11.88 us,
-  // a small greedy one 8.10 -> 7.77, against the same fields spread over the
-  // struct's 600 bytes).
+  // line at a time, and these fill its first two (one row 12.27 -> 11.88 us
+  // against the same fields spread over the struct's 600 bytes, when the
+  // finalizer's fields were loaded at the start too; with late_args the order
+  // of the fields past n_chunks and nslots shows no more: 11.1 us either way).
   int32_t n_chunks, nslots;
   // sample_kernel's grid: rows in groups of 2^xcd_log2 (the device's XCD
   // count, or 1), nrows of them; xcd_test 2 makes the rows of several chunks
@@ -464,7 +465,7 @@ struct Args {
   float* p_max;  // argmax_probs (greedy_all)
   // sparse controls (controls == nullptr: none) and what control_kernel makes
   // of them: per row a patch list of (id << 32 | final value bits) sorted by id,
-  // CTL_MAX entries apart, and the first patch of every chunk (n_chunks + 1
+  // ctl_cap entries apart, and the first patch of every chunk (n_chunks + 1
   // offsets per row)
   const xs_row_control* controls;
   const uint32_t* ctl_ids;
@@ -1703,7 +1704,10 @@ XS_DEV int gather_survivors(const uint64_t* rowrec, int nsp, int nsub, int kp, c
       }
     }
   }
-  if (M > 128) trim();  // (the sort that follows counts, for each entry, all the others)
+  // Up to 128 the finalizer sorts in registers, more by counting, for each
+  // entry, all the others; trimming below that costs more than the sort saves
+  // (24 rows of 33,001 ids at top_k 100: 30.6 us, 32.3 trimmed from 64).
+  if (M > 128) trim();
   return M;
 }
 
@@ -1797,7 +1801,10 @@ XS_DEV bool fin_fast(const Args& a, const Cfg& cfg, int row, int nsub, const Ctl
   // entries past the preloaded ones (a sub-record holding more than EPRE); in
   // a sorted sub-record (flag 4) they end at the first one below the floor.
   // Many of them in one sub-record, or more survivors than the list holds:
-  // the general path's gather_survivors.
+  // the general path's gather_survivors, which reads 256 of them to a round
+  // trip where this loop reads 4 a lane.  (24 masked rows of 64,003 ids at
+  // top_k 63: 32.9 us leaving at more than 16 or 32 entries, 39.3 at 64; 32
+  // masked rows at top_k 50: 27.0 us leaving at 16, 22.1 at 32 and 64.)
   const bool srt = (hf & 4u) != 0;
   int lim = (srt && pk_key(E[EPRE - 1]) < tau) ? EPRE : cnt;
   if (XS_RARE(M > SURV || __ballot(lim > 2 * EPRE))) return false;
@@ -2026,10 +2033,10 @@ XS_DEV bool fin_fast(const Args& a, const Cfg& cfg, int row, int nsub, const Ctl
 
 // ---------------------------------------------------------------------------
 // Row finalize, general case (the rows fin_fast leaves): any number of
-// sub-records up to GMAX * 64, K' up to KSEL, survivors past SURV, sparse
-// controls, and probability ties at the top-k boundary.  Lane l handles
-// sub-records l + 64g; group 0's header words and first EPRE entries are the
-// ones finalize_row preloaded, the rest are read where they are used.
+// sub-records up to GMAX * 64, K' up to KSEL, survivors past SURV, and
+// probability ties at the top-k boundary.  Lane l handles sub-records
+// l + 64g; group 0's header words and first EPRE entries are the ones
+// finalize_row preloaded, the rest are read where they are used.
 template <bool HAS_MASK, bool WANT_LSE, bool HAS_CTL, bool LOC>
 XS_DEV void fin_general(const Args& a, const Cfg cfg, int row, const uint64_t* rowrec,
                         int nsp, int nsub, const float* rowp, const uint32_t* mrow, const CtlRow& cr,
@@ -2899,9 +2906,10 @@ XS_DEV bool deferred(const Cfg& cfg, const FinLds& F) {
 // them; a term the bound leaves open, or a subnormal one, is recomputed
 // correctly rounded.  The row's last workgroup walks the segments in order: a
 // segment whose summary holds s's binade, with no half-way term, and whose
-// units keep s below the next binade adds them to s's bits; any other
-// segment adds units up to its first term that carries or ties, and from
-// there its terms one at a time in f32, as the reference does.  Segments
+// units keep s below the next binade adds them to s's bits; one with a single
+// half-way term adds them and one more where the sum there is odd (one_tie);
+// any other segment adds units up to its first term that carries or ties, and
+// from there its terms one at a time in f32, as the reference does.  Segments
 // where the exact sum may pass a power of two, or that hold a half-way term,
 // keep their correctly rounded terms in a side buffer for that.
 constexpr uint32_t GSAT = 1u << 23;    // grid units that always carry into the next binade
@@ -3907,7 +3915,9 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(4, 8))) v
   // Many more than K' staged (a mask whose few ranges leave the chunk bound
   // weak): only those at or above their K'-th largest go out, so the finalizer
   // reads K' of a wave and not up to CAPW (24 masked rows of 64,003 ids at
-  // top_k 50: 32.7 -> 29.7 us).
+  // top_k 50: 32.7 -> 29.7 us).  From 64 staged entries up: rows 24 x 33,001
+  // at top_k 40 take 16.0 us, 16.6 from 32 (the trim costs more than the
+  // entries) and 19.4 from 128.
   if (XS_RARE(!ovf && cnt > 64 && cnt > kp)) {
     wave_lds_sync();
     uint64_t v[CAPW / 64];
@@ -5775,7 +5785,7 @@ int xcd_placement(int device) {
 
 // One sample_kernel launch over rows x n_chunks workgroups (it finalizes the
 // rows itself), or, for a large batch, sample_kernel then finalize_kernel; a
-// call with sparse controls runs control_kernel (one workgroup per row) first,
+// call with sparse controls runs control_kernel (rows x n_chunks too) first,
 // one that can observe the serial denominator serial_kernel after them, and a
 // context sized for top_k >= 128 the whole-row kernels last.
 template <bool M, bool S, bool C>

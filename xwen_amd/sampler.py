@@ -374,8 +374,10 @@ def cost_order(temperature, top_k, *, controlled=None) -> np.ndarray:
     """A row order for sample_batch that starts the rows with the costliest
     finalization first: stochastic rows by top_k, largest first (above 63 the
     general finalizer runs), then greedy rows; rows with sparse controls
-    (`controlled`, a bool per row) before all others.  Stable, so equal rows
-    keep their order."""
+    (`controlled`, a bool per row), whose draw is also checked against the
+    serial sum, before all others (256 mixed rows of 248,320 ids, a quarter of
+    them controlled: 102.2 us a call, 106.1 ordered by top_k alone, 115.1 in
+    the batch's order).  Stable, so equal rows keep their order."""
     t = np.asarray(temperature, np.float64)
     k = np.asarray(top_k, np.int64)
     rows = max(t.size, k.size)
