@@ -182,10 +182,11 @@ class Context:
                 torch.device("cuda", self.device))
         return cache[key]
 
+    def bind_stream(self, stream):
+        _lib.check(self.lib.xs_set_stream(self.h, C.c_void_p(stream.cuda_stream)), "xs_set_stream")
+
     def bind_current_stream(self):
-        torch = _torch()
-        s = torch.cuda.current_stream(self.device).cuda_stream
-        _lib.check(self.lib.xs_set_stream(self.h, C.c_void_p(s)), "xs_set_stream")
+        self.bind_stream(_torch().cuda.current_stream(self.device))
 
     def close(self):
         if getattr(self, "h", None):
@@ -512,7 +513,7 @@ class Sampler:
         uniforms it draws from and the tokens and statuses it leaves, in pinned
         memory that the kernels read and write in place, so that a call makes
         no copies (4 rows: 89 us a call with three uploads, two allocations and
-        two read-backs, 34 without).  A call that ends with its stream's
+        two read-backs, 31 without).  A call that ends with its stream's
         synchronize leaves its block to the next one (_take_buffers)."""
         torch = _torch()
         host = torch.empty((3, rows), dtype=torch.int32, pin_memory=True)
@@ -523,7 +524,8 @@ class Sampler:
         """A block that no launch reads or writes.  One that a call left in an
         exception (after its launch, or in its wait) may still be in use: it is
         kept until its stream has run dry, and never taken again before."""
-        self._free_stuck(None)
+        if self._stuck:
+            self._free_stuck(None)
         b, self._bufs = self._bufs, None
         if b is None or b["rows"] < rows:
             b = self._buffers(max(rows, self.ctx.max_rows))
@@ -532,8 +534,7 @@ class Sampler:
     def _free_stuck(self, drained):
         """Give back the blocks of interrupted calls whose stream has run dry
         (`drained`: one known to have)."""
-        if self._stuck:
-            self._stuck = [e for e in self._stuck if e[0] != drained and not e[0].query()]
+        self._stuck = [e for e in self._stuck if e[0] != drained and not e[0].query()]
 
     def _row_params(self, rows, device):
         """xs_row_params for every row of a call, kept on the device while the
@@ -587,7 +588,7 @@ class Sampler:
         if ctl is not None and ctl.has_sparse():
             controls = controls_tensor([ctl] * rows, logits.device)
         stream = torch.cuda.current_stream(self.ctx.device)
-        self.ctx.bind_current_stream()
+        self.ctx.bind_stream(stream)
         b = self._take_buffers(rows)
         b["u"][:rows] = u
         host = b["host"]
@@ -598,11 +599,13 @@ class Sampler:
         except BaseException:
             self._stuck.append((stream, b, p))
             raise
-        token, st = b["token"][:rows].astype(np.int64), b["status"][:rows].copy()
+        token, st = b["token"][:rows].astype(np.int64), b["status"][:rows]
+        err = SampleError(st.copy()) if st.any() else None
         self._bufs = b
-        self._free_stuck(stream)
-        if st.any():
-            raise SampleError(st)
+        if self._stuck:
+            self._free_stuck(stream)
+        if err is not None:
+            raise err
         return token
 
     def sample(self, logits, uniforms=None):
