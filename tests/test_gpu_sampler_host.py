@@ -117,3 +117,22 @@ def test_a_call_left_in_an_exception_keeps_its_block(oracle, monkeypatch):
         s.sample(torch.zeros((5, V), device="cuda"), np.zeros(5, np.float32))
     for u, want in ((u1, want1), (u2, want2)):
         assert s.sample(xd, u).tolist() == want and not s._stuck
+
+
+def test_options_per_row(oracle):
+    """Options set to one value a row, on a Sampler of more rows, between calls
+    with numbers: each row draws with its own."""
+    from xwen_amd import sampler as xsm
+    rng = np.random.default_rng(8)
+    opts = xsm.SamplerOptions(temperature=0.7, top_k=20, top_p=0.9)
+    s = xsm.Sampler(opts, [0], V, max_rows=8)
+    x = rng.standard_normal((3, V)).astype(np.float32) * np.float32(2.0)
+    xd, u = torch.as_tensor(x).cuda(), workloads.uniforms(rng, 3)
+    T, K, P = np.array([0.0, 0.6, 1.3]), [20, 50, 5], np.array([0.9, 1.0, 0.5])
+    for t, k, p in [(0.7, 20, 0.9), (T, 20, 0.9), (T, K, P), (1.0, 20, P), (T + 0.1, K, P), (0.7, 20, 0.9)]:
+        opts.temperature, opts.top_k, opts.top_p = t, k, p
+        tt, kk, pp = (np.broadcast_to(np.asarray(a), (3,)) for a in (t, k, p))
+        want = [oracle.sample_controlled(x[r], V, float(tt[r]), int(kk[r]), float(pp[r]), u=float(u[r]),
+                                         sum_mode=oracle.SUM_F64).token for r in range(3)]
+        for _ in range(2):
+            assert s.sample(xd, u).tolist() == want

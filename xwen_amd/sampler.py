@@ -538,12 +538,14 @@ class Sampler:
 
     def _row_params(self, rows, device):
         """xs_row_params for every row of a call, kept on the device while the
-        options stay the same."""
-        key = (self.opts.temperature, self.opts.top_k, self.opts.top_p, device)
+        options stay the same numbers (an option given per row is packed anew)."""
+        o, number = self.opts, (int, float, np.number)
+        if not (isinstance(o.temperature, number) and isinstance(o.top_k, number) and isinstance(o.top_p, number)):
+            return params_tensor(o.temperature, o.top_k, o.top_p, rows, device)
+        key = (o.temperature, o.top_k, o.top_p, device)
         if self._params is None or self._params[0] != key or self._params[1] < rows:
             n = max(rows, self.ctx.max_rows)
-            self._params = (key, n, params_tensor(self.opts.temperature, self.opts.top_k, self.opts.top_p,
-                                                  n, device))
+            self._params = (key, n, params_tensor(o.temperature, o.top_k, o.top_p, n, device))
         return self._params[2]
 
     def encodable(self) -> int:
