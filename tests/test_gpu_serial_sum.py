@@ -218,3 +218,46 @@ def test_verify_block_at_top_p_1(ctx, oracle):
                 break
             want += 1
         assert acc[s] == want, (s, acc[s], want)
+
+
+@pytest.mark.parametrize("shape", ["one", "among", "two"])
+def test_segments_of_half_way_terms(oracle, shape):
+    """Every 256-id segment holds terms made half-way at the running sum's binade:
+    one alone, one between two ordinary terms (the walk adds such a segment by
+    its units and a parity bit), or two (it adds the terms)."""
+    from xwen_amd import sampler as xsm
+    v, rows, seg = 40_003, 8, 256
+    rng = np.random.default_rng({"one": 1, "among": 2, "two": 3}[shape])
+    pool = rng.uniform(-1.3, -0.01, 400_000).astype(np.float32)
+    e = oracle.exp_array(pool)
+    x = np.zeros((rows, 40_004), np.float32)
+    allow = np.zeros((rows, v), bool)
+    for r in range(rows):
+        s = np.float32(1.0)  # id 0: the max, its term 1
+        allow[r, 0] = True
+        made = 0
+        for g in range(1, v // seg):
+            ids = np.sort(rng.choice(np.arange(g * seg, (g + 1) * seg), {"one": 1, "among": 3, "two": 2}[shape], False))
+            for n, i in enumerate(ids):
+                at = int(rng.integers(0, len(pool) - 60_000))
+                q = np.arange(at, at + 60_000)
+                if shape != "among" or n == 1:  # half-way: e an odd number of half grid steps
+                    q = q[np.mod(e[q].astype(np.float64) / np.spacing(s), 1.0) == 0.5]
+                j = int(q[rng.integers(0, len(q))])
+                before = s
+                s = np.float32(s + e[j])
+                made += np.spacing(before) == np.spacing(s)
+                x[r, i] = pool[j]
+                allow[r, i] = True
+        assert made > v // seg // 2
+    mask, U = workloads.pack_mask(allow), workloads.uniforms(rng, rows)
+    ctx = xsm.Context(max_rows=rows, vocab=v)
+    ctx.bind_current_stream()
+    d = run_sample(ctx, x, 1.0, 20, 1.0, U, enc=v, mask=mask, cand_k=20)
+    assert (d["status"] == 0).all()
+    assert _checked(oracle, x, 1.0, 20, 1.0, U, d, enc=v, mask=mask, label=f"half-way {shape}") == rows
+    for r in range(rows):
+        o = oracle.sample_controlled(x[r], v, 1.0, 20, 1.0, u=float(U[r]), sum_mode=oracle.SUM_SEQ_F32,
+                                     ctl=oracle.Ctl(allowed=mask[r]))
+        assert np.float32(d["soft_sum"][r]).view(np.uint32) == np.float32(o.ssum).view(np.uint32), r
+    ctx.close()
